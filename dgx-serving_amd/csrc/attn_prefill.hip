@@ -3,18 +3,18 @@
 // Replaces the reference's fav2::flash_v2_kernel (kernels/attention_flash_v2.cuh:104-259) and, for long query
 // runs, flash_attn2bs_p1(_custom)_kernel (kernels/attention_flash.cuh:28-217).
 //
-// Work decomposition. A half tile is 32 rows: tqh tokens x the GRP q-heads of one KV head (token-major), so every
-// K/V byte a workgroup fetches serves the whole GQA group. A workgroup (8 wave64s) takes two half tiles at once
-// and walks the union of their key ranges: for causal prompts the pair (i, n-1-i), so the keys of the short half
-// are fetched once for both and every workgroup carries the same work (a T=1024 prompt at 8 KV heads is 256 equal
-// workgroups); otherwise two neighbouring half tiles. Work items of
-// one (sequence, KV head) get consecutive indices and are mapped onto one XCD (workgroups are dispatched
-// round-robin over the 8 XCDs), so that head's K/V stays in one L2.
+// Work decomposition. A workgroup holds a tile of rows: tokens x the GRP q-heads of one KV head (token-major), so every
+// K/V byte it fetches serves the whole GQA group. A work item is one tile of consecutive tokens, or, for short causal
+// prompts, the pair of half tiles (i, n-1-i) over the union of their key ranges, so that the keys of the short half are
+// fetched once for both and every workgroup carries about the same work (a T=1024 prompt at 8 KV heads is 256 such
+// workgroups). choose_plan picks the tile and the form from the launch's sizes. Work items of one (sequence, KV head)
+// are mapped onto as few XCDs as the number of heads allows (workgroups are dispatched round-robin over the 8 XCDs), so
+// that head's K/V stays in one L2.
 //
 // Keys are walked in steps of SK keys at absolute positions; each wave takes the NSUB 16-key sub-tiles of its key
 // group in a step (one wave per key group and row group). K and V of a step go from HBM/L2 straight into LDS
 // with gfx950 direct-to-LDS buffer loads (no staging registers; the buffer range makes rows past the last key
-// read as zeros), NS-stage ring, one barrier per step. The LDS rows are unpadded and their 16-byte slots are
+// read as zeros), two stages, one barrier per step. The LDS rows are unpadded and their 16-byte slots are
 // XOR-swizzled by the key (kswz, vswz). Each wave then
 //   * computes S^T = K Q^T for its rows on 16x16x32 MFMA (K fragments from LDS, Q fragments in registers),
 //   * masks (causal / window; a wave-uniform test picks the unmasked fast path) and runs the online softmax in
@@ -35,6 +35,7 @@
 #include "attn_device.h"
 #include "attn_internal.h"
 #include <algorithm>
+#include <atomic>
 #include <climits>
 #include <type_traits>
 
@@ -44,22 +45,26 @@ struct PrefArgs {
     Problem p;
     Partials part;
     int kv_split;      // 0: none
-    int nht;           // half tiles per sequence
+    int nht;           // half tiles (pair) or tiles per sequence
     int nsplit;        // key splits per sequence
-    int tqh;           // tokens per half tile
-    int pair;          // 1: a work item is the half-tile pair (i, nht-1-i); 0: the half tiles (2i, 2i+1)
+    int tqh;           // tokens per half tile (pair) or per tile
+    int pair;          // 1: a work item is the half-tile pair (i, nht-1-i); 0: one tile of all the workgroup's rows
     int nitems;        // work items per (sequence, kv head)
-    int nwg;           // total work items
+    int heads;         // sequences x KV heads
+    int grp;           // q-heads per KV head
     float sl2;         // scale * log2(e)
     int fold;          // 1: fold each XCD's slots (two co-resident workgroups per CU take a long and a short item)
+    int q_al;          // Q is 16-byte aligned
+    int grp_mul;       // ceil(65536 / GRP): rho / GRP = rho * grp_mul >> 16 for rho < 128
+    int ways;          // XCDs that share one KV head's items (> 0), or minus the KV heads that share an XCD; 0: neither
 };
 
-// A workgroup is RG x KG waves. RB: 16-row blocks per wave; RG: row groups (waves splitting the tile's rows); KG:
-// key groups (waves splitting each step's keys); NS: LDS stages; NSUB: 16-key sub-tiles per wave and step.
-// RB = 1: the row groups split the tile's rows (the first half of them on the first half tile).
-template <int HD, int RB, int RG, int KG_, int NS_, int NSUB_>
+// A workgroup is RG x KG waves. RB: 16-row blocks per wave; RG: row groups (waves splitting the tile's rows, the first
+// half of them on a pair's first half tile); KG: key groups (waves splitting each step's keys); NS: LDS stages; NSUB:
+// 16-key sub-tiles per wave and step.
+template <int HD, int RB, int RG, int KG_, int NSUB_>
 struct PrefCfg {
-    static constexpr int KG = KG_, NS = NS_, NW = RG * KG_, NT = NW * 64, NSUB = NSUB_;
+    static constexpr int KG = KG_, NW = RG * KG_, NT = NW * 64, NSUB = NSUB_;
     static constexpr int KT = 16 * NSUB;                 // keys per wave per step (NSUB 16-key sub-tiles)
     static constexpr int SK = KG * KT;                   // keys per step
     static constexpr int RR = RG * RB * 16;              // rows per workgroup tile
@@ -70,22 +75,19 @@ struct PrefCfg {
     static constexpr int SLOTS = HD / 8;                 // 16-byte slots per key row
     static constexpr int ROWB = HD * 2;                  // bytes per key row (16-bit operands)
     static constexpr int HALF = SK * ROWB;               // bytes of one K (or V) step tile
-    static constexpr int STAGE = 2 * HALF;               // K and V of one step
+    static constexpr int NQL = RR * SLOTS / 64 / NW;     // 16-byte Q loads per thread
     static constexpr int NLR = SK * SLOTS / 64;          // 64-slot rows of a step tile (one per wave load)
     static constexpr int NLD = (NLR + NW - 1) / NW;      // 16-byte loads per thread per step (K and V each)
-    static constexpr size_t LDS_TILES = (size_t)NS * STAGE;
+    static constexpr size_t LDS_TILES = (size_t)4 * HALF;  // K stages 0 and 1, V stages 1 and 0
     static constexpr int XSTR = HD / KG + 4;             // merge exchange row stride (floats)
-    // merge exchange of one row block: [row group][owner key group][sender slot (KG-1)][16 rows][XSTR]
-    static constexpr size_t LDS_MERGE = (size_t)RG * KG * (KG - 1) * 16 * XSTR * 4;
+    // merge exchange: [row block][row group][owner key group][sender slot (KG-1)][16 rows][XSTR]
+    static constexpr size_t LDS_MERGE = (size_t)RB * RG * KG * (KG - 1) * 16 * XSTR * 4;
     static constexpr size_t LDS_STATS = (size_t)2 * NW * RB * 16 * 4;
-    static constexpr size_t LDS_MAIN = LDS_TILES > LDS_MERGE ? LDS_TILES : LDS_MERGE;
-    static constexpr size_t STATS_OFF = LDS_MAIN;        // merge statistics past the tiles
-    static constexpr size_t LDS = LDS_MAIN + LDS_STATS;
-    // Waves past the last 64-slot row issue fewer loads; the step wait is then exact only without younger steps in
-    // flight (NS = 2 waits for vmcnt 0).
-    static_assert((SK * SLOTS) % 64 == 0 && (NLR % NW == 0 || NS == 2), "step loads");
-    static_assert(RB == 1 && RG % 2 == 0, "row block layout");
-    static_assert(NS >= 2 && NS <= 4, "stages");
+    static constexpr size_t STATS_OFF = LDS_MERGE;       // merge statistics past the exchange (over the tiles)
+    static constexpr size_t LDS = LDS_TILES > LDS_MERGE + LDS_STATS ? LDS_TILES : LDS_MERGE + LDS_STATS;
+    static_assert((SK * SLOTS) % 64 == 0, "step loads");
+    static_assert((RR * SLOTS) % (64 * NW) == 0 && RR * ROWB <= 2 * HALF && HR % (64 / SLOTS) == 0, "Q tile in a stage");
+    static_assert(RG % 2 == 0 && (NSUB == 2 || (NSUB == 1 && RB == 1)), "row block layout");
     static_assert((KG == 2 || KG == 4) && DB % KG == 0, "key groups");
 };
 
@@ -101,19 +103,31 @@ __device__ __forceinline__ int kswz(int k) { return k & 15; }
 typedef __attribute__((address_space(3))) void lds_void;
 typedef __attribute__((address_space(1))) void glb_void;
 
-// Wait until at most `pending` later steps (PER memory operations each) are still in flight.
-template <int PER>
-__device__ __forceinline__ void wait_steps(int pending) {
-    if (pending >= 2) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(2 * PER) : "memory");
-    else if (pending == 1) asm volatile("s_waitcnt vmcnt(%0)" ::"n"(PER) : "memory");
-    else asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+// LDS reads at addr + OFF that the caller waits for with lds_wait: 16 bytes per lane, and the transpose read.
+template <int OFF> __device__ __forceinline__ void lds_read16(u32x4 &d, unsigned addr) {
+    asm volatile("ds_read_b128 %0, %1 offset:%2" : "=v"(d) : "v"(addr), "n"(OFF) : "memory");
+}
+template <int OFF> __device__ __forceinline__ void lds_read_tr(u32x2 &d, unsigned addr) {
+    asm volatile("ds_read_b64_tr_b16 %0, %1 offset:%2" : "=v"(d) : "v"(addr), "n"(OFF) : "memory");
+}
+// Wait until at most CNT younger LDS reads are in flight; the registers in r are written by older ones.
+template <int CNT, class T, int N>
+__device__ __forceinline__ void lds_wait(T (&r)[N]) {
+    static_assert(N == 2 || N == 4 || N == 8, "read batch");
+    if constexpr (N == 2)
+        asm volatile("s_waitcnt lgkmcnt(%[c])" : "+v"(r[0]), "+v"(r[1]) : [c] "n"(CNT) : "memory");
+    else if constexpr (N == 4)
+        asm volatile("s_waitcnt lgkmcnt(%[c])" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]) : [c] "n"(CNT) : "memory");
+    else
+        asm volatile("s_waitcnt lgkmcnt(%[c])" : "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]), "+v"(r[4]), "+v"(r[5]),
+                     "+v"(r[6]), "+v"(r[7]) : [c] "n"(CNT) : "memory");
 }
 
-template <int HD, int RB, int RG, int KG_, int NS_, int NSUB, int WPE, int KVT, int QT, int OT>
+template <int HD, int RB, int RG, int KG_, int NSUB, int WPE, int KVT, int QT, int OT>
 __global__ void __launch_bounds__(RG * KG_ * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
 prefill_kernel(const PrefArgs a) {
-    using Cf = PrefCfg<HD, RB, RG, KG_, NS_, NSUB>;
-    constexpr int KG = Cf::KG, NS = Cf::NS, SK = Cf::SK, KS = Cf::KS, DB = Cf::DB, NLD = Cf::NLD, DO = Cf::DO;
+    using Cf = PrefCfg<HD, RB, RG, KG_, NSUB>;
+    constexpr int KG = Cf::KG, SK = Cf::SK, KS = Cf::KS, DB = Cf::DB, NLD = Cf::NLD, DO = Cf::DO;
     constexpr int SLOTS = Cf::SLOTS, ROWB = Cf::ROWB, HR = Cf::HR;
     constexpr bool F16 = OpIsF16<KVT>::value;
     constexpr bool DMA = KVT != DT_FP32;                 // 16-bit caches go straight to LDS
@@ -123,18 +137,24 @@ prefill_kernel(const PrefArgs a) {
     float *stm = reinterpret_cast<float *>(smem + Cf::STATS_OFF), *stl = stm + Cf::NW * RB * 16;
 
     const Problem &p = a.p;
-    // XCD-aware work index: dispatch slot b runs on XCD b % 8, and consecutive work items (one KV head's tiles,
-    // longest first) share an XCD, so that head's K/V stays in one L2. With a.fold the local slot k is folded:
-    // slots k and k + per/2 - which the dispatcher places on the same CU when two workgroups fit a CU and the grid
-    // is one round - take the k-th longest and the k-th shortest item.
-    const int per = (int)gridDim.x / 8, k_loc = (int)blockIdx.x / 8, h_loc = (per + 1) / 2;
-    const int w_item = ((int)blockIdx.x % 8) * per + (!a.fold || k_loc < h_loc ? k_loc : per - 1 - (k_loc - h_loc));
-    if (w_item >= a.nwg) return;
-    const int seq = w_item / (p.NKV * a.nitems);
-    const int kvh = (w_item / a.nitems) % p.NKV;
-    const int item = w_item % a.nitems;
-    const int sp = item % a.nsplit, qi = item / a.nsplit;
-    const int GRP = p.NQ / p.NKV;
+    // XCD-aware work index: dispatch slot b runs on XCD b % 8, and the work items of one KV head (longest first) share
+    // an XCD, so that head's K/V stays in one L2. Fewer heads than XCDs: a head's items are dealt in turn to its
+    // `ways` XCDs; a multiple of 8 heads: an XCD takes its heads' items in turn; other counts: every head's longest
+    // items first, over all XCDs. Long items of every head start first in each case: with the longest half of a head on
+    // one XCD and the shortest on another, the 1377-token prompt of 24 q-heads over 4 KV heads took 75 instead of 56 us.
+    // With a.fold the local slot k is folded: slots k and k + per/2 - which the dispatcher places on the same CU when
+    // two workgroups fit a CU and the grid is one round - take the k-th longest and the k-th shortest item.
+    const int per = (int)gridDim.x / 8, k_loc = (int)blockIdx.x / 8, h_loc = (per + 1) / 2, xcd = (int)blockIdx.x % 8;
+    const int k_f = !a.fold || k_loc < h_loc ? k_loc : per - 1 - (k_loc - h_loc);
+    int head, item;                                                     // head = sequence * NKV + KV head
+    if (a.ways > 0) { head = xcd / a.ways; item = k_f * a.ways + xcd % a.ways; }
+    else if (a.ways < 0) { item = k_f / -a.ways; head = xcd + 8 * (k_f + item * a.ways); }
+    else { const int i = 8 * k_f + xcd; item = i / a.heads; head = i - item * a.heads; }
+    if (item >= a.nitems || head >= a.heads) return;
+    // (runtime divisions take ~200 cycles each: skipped where the launch makes them trivial)
+    const int seq = p.nseq > 1 ? head / p.NKV : 0, kvh = head - seq * p.NKV;
+    const int qi = a.nsplit > 1 ? item / a.nsplit : item, sp = item - qi * a.nsplit;
+    const int GRP = a.grp;
 
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, ln = lane & 15;
     const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
@@ -145,11 +165,8 @@ prefill_kernel(const PrefArgs a) {
     // Prefill tokens are consecutive: token t of this sequence sits at position pbase + t.
     const int pbase = __builtin_amdgcn_readfirstlane(p.pos_arr ? p.pos_arr[seq] : p.base);
 
-    // The two half tiles of this work item (longest first) and their tokens; an empty half has tok1 == tok0.
-    const int nhalf_items = a.nitems / a.nsplit;
-    int ht0, ht1;
-    if (a.pair) { ht0 = a.nht - 1 - qi; ht1 = qi < ht0 ? qi : -1; }
-    else { const int i2 = nhalf_items - 1 - qi; ht0 = 2 * i2 + 1 < a.nht ? 2 * i2 + 1 : 2 * i2; ht1 = 2 * i2 + 1 < a.nht ? 2 * i2 : -1; }
+    // The work item's tokens: one tile, or two half tiles (longest first; an empty half has tok1 == tok0).
+    const int ht0 = a.nht - 1 - qi, ht1 = a.pair && qi < ht0 ? qi : -1;
     int tok0[2], tok1[2];
     tok0[0] = ht0 * a.tqh; tok1[0] = min(p.T, tok0[0] + a.tqh);
     tok0[1] = ht1 < 0 ? 0 : ht1 * a.tqh; tok1[1] = ht1 < 0 ? 0 : min(p.T, tok0[1] + a.tqh);
@@ -161,62 +178,72 @@ prefill_kernel(const PrefArgs a) {
     if (a.kv_split > 0) { j_lo = max(j_lo, sp * a.kv_split); j_hi = min(j_hi, (sp + 1) * a.kv_split); }
     const int s0 = j_lo / SK, nsteps = j_lo < j_hi ? (j_hi - 1) / SK - s0 + 1 : 0;
 
-    // Step loads: thread slot S = (wave*NLD + u)*64 + lane of the K (V) half of a stage holds the 16-byte column
-    // (S % SLOTS) ^ kswz(key) (vswz(key)) of key row key = S / SLOTS; its byte offset from the step's first key row
-    // is fixed.
+    // Step loads: thread slot S = (wave*NLD + u)*64 + lane of a K (V) stage holds the 16-byte column
+    // (S % SLOTS) ^ kswz(key) (vswz(key)) of key row key = S / SLOTS, at a fixed byte offset from the step's first key
+    // row. With a power of two of rows per wave, slot u's key is a bitwise or of the row of slot 0 and u * RPL, so its
+    // swizzle is that of slot 0 XOR a constant: two registers hold a wave's offsets instead of 2 NLD.
     const unsigned krow_b = (unsigned)(krow * sizeof(KE));
-    unsigned ld_koff[NLD], ld_voff[NLD];
+    constexpr int RPL = 64 / SLOTS;                      // key rows of one 64-slot load
+    constexpr bool XORU = ((NLD * RPL) & (NLD * RPL - 1)) == 0 && Cf::NLR % Cf::NW == 0;
+    unsigned ld_koff[XORU ? 1 : NLD], ld_voff[XORU ? 1 : NLD];
 #pragma unroll
-    for (int u = 0; u < NLD; u++) {
+    for (int u = 0; u < (XORU ? 1 : NLD); u++) {
         const int S = (wave * NLD + u) * 64 + lane, key = S / SLOTS;
-        ld_koff[u] = (unsigned)key * krow_b + (unsigned)(((S % SLOTS) ^ kswz(key)) * 8 * sizeof(KE));
-        ld_voff[u] = (unsigned)key * krow_b + (unsigned)(((S % SLOTS) ^ vswz(key)) * 8 * sizeof(KE));
+        ld_koff[u] = (unsigned)(((S % SLOTS) ^ kswz(key)) * 8 * sizeof(KE)) + (XORU ? 0u : (unsigned)key * krow_b);
+        ld_voff[u] = (unsigned)(((S % SLOTS) ^ vswz(key)) * 8 * sizeof(KE)) + (XORU ? 0u : (unsigned)key * krow_b);
     }
-    // Step k of the walk into stage k % NS. Keys past the last position re-read that position (they are masked), so
+    const unsigned ld_row = XORU ? (unsigned)(wave * NLD * RPL + lane / SLOTS) * krow_b : 0u;
+    auto k_off = [&](int u) -> unsigned {
+        if constexpr (XORU) return (ld_koff[0] ^ (unsigned)(kswz(u * RPL) * 8 * sizeof(KE))) + u * RPL * krow_b;
+        else return ld_koff[u];
+    };
+    auto v_off = [&](int u) -> unsigned {
+        if constexpr (XORU) return (ld_voff[0] ^ (unsigned)(vswz(u * RPL) * 8 * sizeof(KE))) + u * RPL * krow_b;
+        else return ld_voff[u];
+    };
+    // Step k of the walk into stage k % 2. Keys past the last position re-read that position (they are masked), so
     // every load is in bounds; only a step that crosses the end needs the clamped addresses.
     // Loads [u0, u1) of the thread's NLD slots (K and V each).
     // 16-bit caches: buffer loads straight into LDS over the byte range the workgroup may read (the ring, or the
     // keys below hi_b), so the rows past the last key of a step read as zeros (they are masked) without clamping.
     const uint32_t kv_bytes = p.kv_cap > 0 ? (uint32_t)p.kv_cap * krow_b
                                            : (uint32_t)(max(hi_b, 1) - 1) * krow_b + (uint32_t)(HD * sizeof(KE));
+    const __amdgpu_buffer_rsrc_t krs = make_rsrc(Kb, kv_bytes), vrs = make_rsrc(Vb, kv_bytes);
     int it_cur = 0;                                                     // the step being computed
-    // Step k < 0 is a no-op step: every lane is out of range, so its loads write zeros into the stage of the step
-    // before (already consumed by every wave) and touch no memory; this keeps the issue points branch-free.
-    // prep(k) forms a step's buffer descriptors and stage once; issue_part(st, u0, u1) issues slots [u0, u1).
-    struct StepLd { __amdgpu_buffer_rsrc_t krs, vrs; unsigned char *kd; int s, soff; };
+    // Step k < 0 is a no-op step: every lane is out of range, so its loads write zeros into the stages of the step
+    // after (already consumed by every wave) and touch no memory; this keeps the issue points branch-free.
+    // prep(k) forms a step's first byte offset and stages; issue_part(st, u0, u1) issues slots [u0, u1).
+    struct StepLd { unsigned char *kd, *vd; unsigned soff; int s; };
     auto prep = [&](int k) {
         StepLd st;
-        st.s = s0 + (k < 0 ? 0 : k);
-        st.kd = smem + (size_t)((k < 0 ? it_cur + 1 : k) % NS) * Cf::STAGE;
-        st.soff = __builtin_amdgcn_readfirstlane(key_row(p, st.s * SK) * (int)krow_b);
-        // the step's rows as the buffer (the range check covers the vector offset only)
-        const uint32_t left = k < 0 || (uint32_t)st.soff >= kv_bytes ? 0u : kv_bytes - (uint32_t)st.soff;
-        st.krs = make_rsrc(reinterpret_cast<const char *>(Kb) + st.soff, left);
-        st.vrs = make_rsrc(reinterpret_cast<const char *>(Vb) + st.soff, left);
+        const int kst = k < 0 ? it_cur + 1 : k;
+        st.s = s0 + kst;
+        st.kd = smem + (size_t)(kst % 2) * Cf::HALF;
+        st.vd = smem + (size_t)(3 - kst % 2) * Cf::HALF;
+        // (the range check covers the vector offset, which holds the step's offset too)
+        st.soff = k < 0 ? kv_bytes : (unsigned)__builtin_amdgcn_readfirstlane((int)((unsigned)key_row(p, st.s * SK) * krow_b));
         return st;
     };
     auto issue_part = [&](const StepLd &st, int u0, int u1) {
-        const int s = st.s, soff = st.soff;
-        unsigned char *kd = st.kd, *vd = kd + Cf::HALF;
+        const unsigned row = ld_row + st.soff;
 #pragma unroll
         for (int u = 0; u < NLD; u++) {
             if (u < u0 || u >= u1) continue;
             const int i = wave * NLD + u;
             if (Cf::NLR % Cf::NW != 0 && i >= Cf::NLR) continue;       // wave-uniform: past the tile
+            unsigned koff = k_off(u) + row, voff = v_off(u) + row;
             if constexpr (!DMA) {
-                const char *ks = reinterpret_cast<const char *>(Kb) + soff;
-                const char *vs = reinterpret_cast<const char *>(Vb) + soff;
-                unsigned koff = ld_koff[u], voff = ld_voff[u];
+                if (st.soff >= kv_bytes) continue;
                 const int S = i * 64 + lane;
-                if (s * SK + SK > hi_b) {
-                    const unsigned key = (unsigned)(S / SLOTS), lim = (unsigned)(hi_b - 1 - s * SK);
+                if (st.s * SK + SK > hi_b) {
+                    const unsigned key = (unsigned)(S / SLOTS), lim = (unsigned)(hi_b - 1 - st.s * SK);
                     if (key > lim) { koff -= (key - lim) * krow_b; voff -= (key - lim) * krow_b; }
                 }
-                *reinterpret_cast<u32x4 *>(kd + (size_t)S * 16) = load8_op<KVT, F16>(reinterpret_cast<const KE *>(ks + koff));
-                *reinterpret_cast<u32x4 *>(vd + (size_t)S * 16) = load8_op<KVT, F16>(reinterpret_cast<const KE *>(vs + voff));
+                *reinterpret_cast<u32x4 *>(st.kd + (size_t)S * 16) = load8_op<KVT, F16>(reinterpret_cast<const KE *>(reinterpret_cast<const char *>(Kb) + koff));
+                *reinterpret_cast<u32x4 *>(st.vd + (size_t)S * 16) = load8_op<KVT, F16>(reinterpret_cast<const KE *>(reinterpret_cast<const char *>(Vb) + voff));
             } else {
-                buffer_load_lds16(st.krs, kd + (size_t)i * 1024, (int)ld_koff[u]);
-                buffer_load_lds16(st.vrs, vd + (size_t)i * 1024, (int)ld_voff[u]);
+                buffer_load_lds16(krs, st.kd + (size_t)i * 1024, (int)koff);
+                buffer_load_lds16(vrs, st.vd + (size_t)i * 1024, (int)voff);
             }
         }
     };
@@ -228,43 +255,62 @@ prefill_kernel(const PrefArgs a) {
     auto issue_pt = [&](const StepLd &st, int pt) { issue_part(st, pt * PPART, min(NLD, (pt + 1) * PPART)); };
     if (nsteps > 0) issue(0);
 
-    // This wave's row blocks: block rb covers rows [lrow[rb], lrow[rb] + 16) of half tile hb[rb]. Q fragments and
-    // positions per row (an invalid row has pos = -1 and attends nothing), and the wave-uniform key span of each
-    // block (positions grow with the row's token).
-    int htok[RB], hrows[RB], lrow[RB];
+    // The Q tile goes through LDS as well (16 bytes per lane of whole rows, where fragment loads straight from memory
+    // touch 64 bytes of 16 rows each), in the stage that step 1 will fill, in the K layout: 16-byte column c of tile row R
+    // in slot c ^ kswz(R), rows past the last as zeros. Row rho of a half tile is token rho / GRP, head rho % GRP.
+    unsigned char *qs = smem + Cf::HALF;
+    auto tok_of = [&](int rho) { return (int)((unsigned)(rho * a.grp_mul) >> 16); };    // rho / GRP
+    {
+        constexpr bool QDMA = QT != DT_FP32;
+        f32x4 raw[QDMA ? 1 : Cf::NQL][2];
+#pragma unroll
+        for (int u = 0; u < Cf::NQL; u++) {
+            const int i = wave * Cf::NQL + u, hb = a.pair && i * RPL >= HR ? 1 : 0;
+            const int R = i * RPL + lane / SLOTS, rho = R - hb * HR, nr = (tok1[hb] - tok0[hb]) * GRP;
+            const int off = (rho + tok_of(rho) * (p.NQ - GRP)) * HD + ((lane % SLOTS) ^ kswz(R)) * 8;
+            const QE *qb = reinterpret_cast<const QE *>(p.Q) + ((size_t)(seq * p.T + tok0[hb]) * p.NQ + kvh * GRP) * HD;
+            if (QDMA && !a.q_al) {                                      // Q off a 16-byte boundary: through registers
+                u32x4 v = u32x4{0u, 0u, 0u, 0u};
+                if (rho < nr) v = *reinterpret_cast<const u32x4 *>(qb + off);
+                *reinterpret_cast<u32x4 *>(qs + (size_t)i * 1024 + lane * 16) = v;
+            } else if constexpr (QDMA) {
+                const __amdgpu_buffer_rsrc_t qr = make_rsrc(qb, (uint32_t)((nr + tok_of(max(nr - 1, 0)) * (p.NQ - GRP)) * HD * 2));
+                buffer_load_lds16(qr, qs + (size_t)i * 1024, rho < nr ? off * 2 : -16);
+            } else {
+                raw[u][0] = raw[u][1] = f32x4{0.f, 0.f, 0.f, 0.f};
+                if (rho < nr) {
+                    raw[u][0] = *reinterpret_cast<const f32x4 *>(qb + off);
+                    raw[u][1] = *reinterpret_cast<const f32x4 *>(qb + off + 4);
+                }
+            }
+        }
+        if constexpr (!QDMA)
+#pragma unroll
+            for (int u = 0; u < Cf::NQL; u++) {
+                const f32x4 x = raw[u][0], y = raw[u][1];
+                *reinterpret_cast<u32x4 *>(qs + (size_t)(wave * Cf::NQL + u) * 1024 + lane * 16) =
+                    u32x4{pack2<F16>(x.x, x.y), pack2<F16>(x.z, x.w), pack2<F16>(y.x, y.y), pack2<F16>(y.z, y.w)};
+            }
+    }
+    // This wave's row blocks: block rb covers rows [lrow[rb], lrow[rb] + 16) of half tile hb. Positions per row (an invalid
+    // row has pos = -1 and attends nothing), and the wave-uniform key span of each block (positions grow with the row's
+    // token).
+    const int hb = a.pair ? rg * RB * 16 / HR : 0;
+    const int htok = tok0[hb], hrows = (tok1[hb] - tok0[hb]) * GRP;
+    int lrow[RB], rpos[RB];
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
-        const int hb = (rg * 16) / HR;
-        lrow[rb] = rg * 16 - hb * HR;
-        htok[rb] = hb ? tok0[1] : tok0[0];
-        hrows[rb] = (hb ? tok1[1] - tok0[1] : tok1[0] - tok0[0]) * GRP;
+        lrow[rb] = rg * RB * 16 + rb * 16 - hb * HR;
+        rpos[rb] = lrow[rb] + ln < hrows ? pbase + htok + tok_of(lrow[rb] + ln) : -1;
     }
-    int rpos[RB], rlo[RB];
-    u32x4 qop[RB][KS];
-#pragma unroll
-    for (int rb = 0; rb < RB; rb++) {
-        const int rho = lrow[rb] + ln;
-        const bool valid = rho < hrows[rb];
-        const int t = htok[rb] + (valid ? rho / GRP : 0), h = kvh * GRP + (valid ? rho % GRP : 0);
-        const int ps = pbase + t;
-        rpos[rb] = valid ? ps : -1;
-        rlo[rb] = win_lo(ps, p.window);
-        const QE *qrow = reinterpret_cast<const QE *>(p.Q) + ((size_t)(seq * p.T + t) * p.NQ + h) * HD + 8 * g;
-#pragma unroll
-        for (int ks = 0; ks < KS; ks++) qop[rb][ks] = valid ? load8_op<QT, F16>(qrow + 32 * ks) : u32x4{0u, 0u, 0u, 0u};
-    }
-    // Steps 1..NS-2 go out after the Q loads, so that waiting for step it never waits for younger steps.
-#pragma unroll
-    for (int k = 1; k < NS - 1; k++)
-        if (k < nsteps) issue(k);
     int wlo[RB], whi[RB], lo_max[RB], pos_min[RB];
     int wlo_all = INT_MAX, whi_all = -1;
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
-        const int rho1 = min(hrows[rb], lrow[rb] + 16);
+        const int rho1 = min(hrows, lrow[rb] + 16);
         wlo[rb] = INT_MAX; whi[rb] = -1; lo_max[rb] = 0; pos_min[rb] = INT_MAX;
         if (lrow[rb] < rho1) {
-            const int pf = pbase + htok[rb] + lrow[rb] / GRP, pl = pbase + htok[rb] + (rho1 - 1) / GRP;
+            const int pf = pbase + htok + tok_of(lrow[rb]), pl = pbase + htok + tok_of(rho1 - 1);
             wlo[rb] = max(win_lo(pf, p.window), j_lo); whi[rb] = min(pl, j_hi - 1);
             lo_max[rb] = win_lo(pl, p.window); pos_min[rb] = pf;
         }
@@ -277,8 +323,20 @@ prefill_kernel(const PrefArgs a) {
     for (int rb = 0; rb < RB; rb++) {
         m[rb] = kNegInf; l[rb] = 0.f;
 #pragma unroll
-        for (int db = 0; db < DB; db++) acc[rb][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+        for (int db = 0; db < DB; db++) {
+            acc[rb][db] = f32x4{0.f, 0.f, 0.f, 0.f};
+            asm volatile("" : "+v"(acc[rb][db]));                       // cleared here, under the loads, not after the wait
+        }
     }
+    // Q fragments: lane (row ln, group g) holds dims 32 ks + 8 g .. of its rows.
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    u32x4 qop[RB][KS];
+#pragma unroll
+    for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+        for (int ks = 0; ks < KS; ks++)
+            qop[rb][ks] = *reinterpret_cast<const u32x4 *>(qs + (rg * RB * 16 + rb * 16 + ln) * ROWB + (((4 * ks + g) ^ kswz(ln)) << 4));
 
     // Per-lane LDS byte addresses inside a step stage (the key group's rows start at kg*KT). A slot index
     // occupies address bits 4.., and the row base has those bits clear, so "slot s ^ x" is an XOR on the
@@ -287,96 +345,94 @@ prefill_kernel(const PrefArgs a) {
     const unsigned lds0 = (unsigned)(uintptr_t)smem;
     const int vr = 4 * g + (ln >> 2);
     const unsigned kaddr = lds0 + (kg * Cf::KT + ln) * ROWB + ((g ^ kswz(ln)) << 4);
-    const unsigned vaddr = lds0 + Cf::HALF + (kg * Cf::KT + vr) * ROWB + 8 * (ln & 1) + ((((ln & 3) >> 1) ^ vswz(vr)) << 4);
+    const unsigned vaddr = lds0 + 3 * Cf::HALF + (kg * Cf::KT + vr) * ROWB + 8 * (ln & 1) + ((((ln & 3) >> 1) ^ vswz(vr)) << 4);
 
-    // One step's work for the row blocks in ACT (a wave-uniform bit mask). QK: the K fragments of a sub-tile are
-    // read in batches of 4 k-steps (inline asm, one wait per batch, so the reads are not serialised behind the
-    // MFMAs) and each active row block runs its MFMA chain on them. Then one softmax update, then PV with V^T
-    // fragments in batches of 8 transpose reads. A block left out keeps its state exactly (it attends no key).
-    auto step = [&](const int ACT, int jw, unsigned stage, const StepLd &nxt) {
+    // One step's work for this wave's row blocks: qk_softmax, then pv. QK: the K fragments of a sub-tile are read in batches (inline asm,
+    // one wait per batch, so the reads are not serialised behind the MFMAs) and every row block runs its MFMA chain on
+    // them. Then one softmax update, then PV with V^T fragments in batches of transpose reads. A row that attends none
+    // of the step's keys keeps its state exactly. Each issues half of the next step's loads.
+    PFrag<F16> pop[NSUB][RB];
+    auto qk_softmax = [&](int it, const StepLd &nxt) {
         int pt = 0;
+        const int jw = (s0 + it) * SK + kg * Cf::KT;
         // Per-lane LDS bases, made opaque so that the XOR-swizzled fragment addresses are formed next to their
         // reads instead of being hoisted out of the step loop (which held ~30 address registers live and spilled).
-        unsigned kbase = kaddr + stage, vbase = vaddr + stage;
-        asm volatile("" : "+v"(kbase), "+v"(vbase));
-        f32x4 s[NSUB][RB], s2[NSUB][RB];
+        unsigned kbase = kaddr + (it & 1) * Cf::HALF;
+        asm volatile("" : "+v"(kbase));
+        constexpr int NCH = NSUB == 1 ? 2 : 1;                          // independent MFMA chains per S fragment
+        f32x4 s[NSUB][RB][NCH];
 #pragma unroll
         for (int sub = 0; sub < NSUB; sub++)
 #pragma unroll
-            for (int rb = 0; rb < RB; rb++) s[sub][rb] = s2[sub][rb] = f32x4{0.f, 0.f, 0.f, 0.f};
+            for (int rb = 0; rb < RB; rb++)
+#pragma unroll
+                for (int ch = 0; ch < NCH; ch++) s[sub][rb][ch] = f32x4{0.f, 0.f, 0.f, 0.f};
         {
-            // Software-pipelined: batch b = k-steps 2b, 2b+1 of every sub-tile (4 reads at NSUB = 2); batch b+1 is
-            // read before batch b's MFMAs, so the LDS latency hides under them (4 independent MFMA chains).
-            constexpr int KPB = 2, NB = KS / KPB, RPB = KPB * NSUB;
-            static_assert(RPB == 4 || RPB == 2, "batch size");
-            u32x4 kb[2][RPB];
-            auto rd = [&](int b, u32x4 (&dst)[RPB]) {
-#pragma unroll
-                for (int sub = 0; sub < NSUB; sub++)
-#pragma unroll
-                    for (int kk = 0; kk < KPB; kk++)
-                        asm volatile("ds_read_b128 %0, %1" : "=v"(dst[sub * KPB + kk])
-                                     : "v"((kbase + sub * 16 * ROWB) ^ (64u * (b * KPB + kk))) : "memory");
+            // Software-pipelined: batch b = KPB k-steps of every sub-tile; QD batches are read ahead of their MFMAs, so
+            // the LDS latency hides under them. The swizzle XORs the low four bits of a row's slot index, so the four
+            // k-steps that differ there take an XOR of the base and the others an immediate offset.
+            constexpr int KPB = RB == 1 ? 2 : 1, NB = KS / KPB, RPB = KPB * NSUB, QD = 2, NHI = KS / 4;
+            auto ks_of = [](int o) { return (o % NHI) * 4 + o / NHI; };     // k-steps in reading order
+            u32x4 kb[QD][RPB];
+            auto rd = [&](auto b_c) {
+                constexpr int b = decltype(b_c)::value;
+                static_for<KPB>([&](auto kk_c) {
+                    constexpr int kk = decltype(kk_c)::value, o = b * KPB + kk;
+                    const unsigned kx = kbase ^ (64u * (o / NHI));
+                    static_for<NSUB>([&](auto sub_c) {
+                        constexpr int sub = decltype(sub_c)::value;
+                        lds_read16<256 * (o % NHI) + sub * 16 * ROWB>(kb[b % QD][sub * KPB + kk], kx);
+                    });
+                });
             };
-            rd(0, kb[0]);
-#pragma unroll
-            for (int b = 0; b < NB; b++) {
-                u32x4 (&cur)[RPB] = kb[b & 1];
-                if (b + 1 < NB) {
-                    rd(b + 1, kb[(b + 1) & 1]);
-                    if constexpr (RPB == 4)
-                        asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(cur[0]), "+v"(cur[1]), "+v"(cur[2]), "+v"(cur[3])::"memory");
-                    else
-                        asm volatile("s_waitcnt lgkmcnt(2)" : "+v"(cur[0]), "+v"(cur[RPB - 1])::"memory");
-                } else {
-                    if constexpr (RPB == 4)
-                        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(cur[0]), "+v"(cur[1]), "+v"(cur[2]), "+v"(cur[3])::"memory");
-                    else
-                        asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(cur[0]), "+v"(cur[RPB - 1])::"memory");
-                }
+            static_for<QD - 1>([&](auto b_c) { rd(b_c); });
+            static_for<NB>([&](auto b_c) {
+                constexpr int b = decltype(b_c)::value, ahead = b + QD - 1 < NB ? QD - 1 : NB - 1 - b;
+                if constexpr (b + QD - 1 < NB) rd(std::integral_constant<int, b + QD - 1>{});
+                lds_wait<ahead * RPB>(kb[b % QD]);
                 if (b == 0 || b == NB / 2) issue_pt(nxt, pt++);
 #pragma unroll
-                for (int sub = 0; sub < NSUB; sub++)
+                for (int kk = 0; kk < KPB; kk++)
 #pragma unroll
-                    for (int kk = 0; kk < KPB; kk++) {
-                        if (kk & 1) s2[sub][0] = mfma16<F16>(cur[sub * KPB + kk], qop[0][b * KPB + kk], s2[sub][0]);
-                        else s[sub][0] = mfma16<F16>(cur[sub * KPB + kk], qop[0][b * KPB + kk], s[sub][0]);
-                    }
-            }
+                    for (int sub = 0; sub < NSUB; sub++)
+#pragma unroll
+                        for (int rb = 0; rb < RB; rb++)
+                            s[sub][rb][kk % NCH] = mfma16<F16>(kb[b % QD][sub * KPB + kk], qop[rb][ks_of(b * KPB + kk)], s[sub][rb][kk % NCH]);
+            });
         }
         float tv[NSUB][RB][4], mnew[RB];
         bool need = false;
 #pragma unroll
         for (int rb = 0; rb < RB; rb++) {
-            mnew[rb] = m[rb];
-            if (!((ACT >> rb) & 1)) continue;
             const bool full = jw >= j_lo && jw + Cf::KT <= j_hi && jw >= lo_max[rb] && jw + Cf::KT - 1 <= pos_min[rb];
             float mx = kNegInf;
 #pragma unroll
             for (int sub = 0; sub < NSUB; sub++) {
-                const f32x4 sc = (s[sub][rb] + s2[sub][rb]) * a.sl2;
+                f32x4 sc = s[sub][rb][0];
+                if constexpr (NCH == 2) sc += s[sub][rb][1];
+                sc *= a.sl2;
 #pragma unroll
                 for (int i = 0; i < 4; i++) tv[sub][rb][i] = sc[i];
             }
             if (!full) {                                        // one wave-uniform test; per key only off the fast path
+                const int kl = max(j_lo, win_lo(rpos[rb], p.window)) - jw - 4 * g, kh = min(j_hi - 1, rpos[rb]) - jw - 4 * g;
 #pragma unroll
                 for (int sub = 0; sub < NSUB; sub++)
 #pragma unroll
-                    for (int i = 0; i < 4; i++) {
-                        const int key = jw + 16 * sub + 4 * g + i;
-                        if (!(key >= j_lo && key < j_hi && key >= rlo[rb] && key <= rpos[rb])) tv[sub][rb][i] = kNegInf;
-                    }
+                    for (int i = 0; i < 4; i++)
+                        if ((16 * sub + i < kl) | (16 * sub + i > kh)) tv[sub][rb][i] = kNegInf;
             }
 #pragma unroll
             for (int sub = 0; sub < NSUB; sub++)
 #pragma unroll
                 for (int i = 0; i < 4; i++) mx = fmaxf(mx, tv[sub][rb][i]);
             mx = max_over_groups(mx);
-            if (mx > m[rb] + kRescaleThreshold) { mnew[rb] = mx; need = true; }
+            mnew[rb] = mx > m[rb] + kRescaleThreshold ? mx : m[rb];
+            need |= mnew[rb] != m[rb];
         }
         if (__any(need)) {
-            // every block (an inactive one has mnew == m, alpha = 1): a per-block condition here made the compiler
-            // keep two copies of the accumulator
+            // every block (an unmoved one has alpha = 1): a per-block condition here made the compiler keep two copies
+            // of the accumulator
 #pragma unroll
             for (int rb = 0; rb < RB; rb++) {
                 const float alpha = (mnew[rb] == m[rb]) ? 1.f : fast_exp2(m[rb] - mnew[rb]);
@@ -385,85 +441,75 @@ prefill_kernel(const PrefArgs a) {
                 for (int db = 0; db < DB; db++) acc[rb][db] *= alpha;
             }
         }
-        while (pt < 3) issue_pt(nxt, pt++);
-        PFrag<F16> pop[NSUB][RB];
 #pragma unroll
-        for (int sub = 0; sub < NSUB; sub++)
+        for (int rb = 0; rb < RB; rb++) {
+            const float mr = m[rb] == kNegInf ? 0.f : m[rb];    // no key seen yet: every score is -inf, exp2 gives 0
 #pragma unroll
-            for (int rb = 0; rb < RB; rb++) {
-                if (!((ACT >> rb) & 1)) { pop[sub][rb] = PFrag<F16>{u32x2{0u, 0u}, u32x2{0u, 0u}}; continue; }
+            for (int sub = 0; sub < NSUB; sub++) {
                 float pv[4];
 #pragma unroll
-                for (int i = 0; i < 4; i++) pv[i] = (tv[sub][rb][i] == kNegInf) ? 0.f : fast_exp2(tv[sub][rb][i] - m[rb]);
+                for (int i = 0; i < 4; i++) pv[i] = fast_exp2(tv[sub][rb][i] - mr);
                 l[rb] += (pv[0] + pv[1]) + (pv[2] + pv[3]);
                 pop[sub][rb] = p_frag<F16>(pv[0], pv[1], pv[2], pv[3]);
             }
-        if constexpr (NSUB == 2) {
-            // PV on 16x16x32 over both sub-tiles at once (the order of keys inside an MFMA's reduction is free):
-            // k-group g of the MFMA holds keys 4g..4g+3 of sub-tile 0 and then of sub-tile 1, which is what the
-            // lane's two S^T fragments hold (B operand = the two P^T halves) and what two transpose reads of V give
-            // (A operand). Software-pipelined: batch b = 4 dim blocks (8 reads); batch b+1 is read before batch b's
-            // MFMAs.
-            constexpr int PB = 4, NPB = DB / PB;
-            u32x2 vb2[2][2 * PB];
-            auto rdv = [&](int b, u32x2 (&dst)[2 * PB]) {
-#pragma unroll
-                for (int j = 0; j < PB; j++)
-#pragma unroll
-                    for (int sub = 0; sub < 2; sub++)
-                        asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(dst[2 * j + sub])
-                                     : "v"((vbase + sub * 16 * ROWB) ^ (32u * (b * PB + j))) : "memory");
-            };
-            rdv(0, vb2[0]);
-#pragma unroll
-            for (int b = 0; b < NPB; b++) {
-                u32x2 (&cur)[2 * PB] = vb2[b & 1];
-                if (b + 1 < NPB) {
-                    rdv(b + 1, vb2[(b + 1) & 1]);
-                    asm volatile("s_waitcnt lgkmcnt(8)" : "+v"(cur[0]), "+v"(cur[1]), "+v"(cur[2]), "+v"(cur[3]), "+v"(cur[4]),
-                                 "+v"(cur[5]), "+v"(cur[6]), "+v"(cur[7])::"memory");
-                } else {
-                    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(cur[0]), "+v"(cur[1]), "+v"(cur[2]), "+v"(cur[3]), "+v"(cur[4]),
-                                 "+v"(cur[5]), "+v"(cur[6]), "+v"(cur[7])::"memory");
-                }
-#pragma unroll
-                for (int j = 0; j < PB; j++)
-                    acc[0][b * PB + j] = mfma_pv32_hi<F16>(u32x4{cur[2 * j][0], cur[2 * j][1], cur[2 * j + 1][0], cur[2 * j + 1][1]},
-                                                           pop[0][0], pop[1][0], acc[0][b * PB + j]);
-#pragma unroll
-                for (int j = 0; j < PB; j++)
-                    acc[0][b * PB + j] = mfma_pv32_lo<F16>(u32x4{cur[2 * j][0], cur[2 * j][1], cur[2 * j + 1][0], cur[2 * j + 1][1]},
-                                                           pop[0][0], pop[1][0], acc[0][b * PB + j]);
-                if (pt < NPART && b % 2 == 1) issue_pt(nxt, pt++);
-            }
         }
-        if constexpr (NSUB != 2) {
-            // Software-pipelined PV: batch b = 4 dim blocks of one sub-tile; batch b+1 is read before batch b's MFMAs.
-            constexpr int PB = 4, NPB = NSUB * DB / PB;
-            u32x2 vb2[2][PB];
-            auto rdv = [&](int b, u32x2 (&dst)[PB]) {
-                const int sub = b / (DB / PB), d0 = (b % (DB / PB)) * PB;
+    };
+    auto pv = [&](int it, const StepLd &nxt) {
+        int pt = NPART / 2;
+        unsigned vbase = vaddr - (it & 1) * Cf::HALF;
+        asm volatile("" : "+v"(vbase));
+        // PV with V^T fragments in batches of PB dim blocks, software-pipelined: batch b+1 is read before batch b's MFMAs.
+        // As for K, the eight dim blocks that differ in the swizzled bits take an XOR of the base, the others (16-byte
+        // slots 16 apart) an immediate offset.
+        // NSUB == 2: PV on 16x16x32 over both sub-tiles at once (the order of keys inside an MFMA's reduction is free):
+        // k-group g of the MFMA holds keys 4g..4g+3 of sub-tile 0 and then of sub-tile 1, which is what the lane's two
+        // S^T fragments hold (B operand = the two P^T halves) and what two transpose reads of V give (A operand).
+        constexpr int PB = RB == 1 ? 4 : 2, NPB = DB / PB, NHV = DB / 8;
+        auto db_of = [](int o) { return (o % NHV) * 8 + o / NHV; };         // dim blocks in reading order
+        u32x2 vb2[2][NSUB * PB];
+        auto rdv = [&](auto b_c) {
+            constexpr int b = decltype(b_c)::value;
+            static_for<PB>([&](auto j_c) {
+                constexpr int j = decltype(j_c)::value, o = b * PB + j;
+                const unsigned vx = vbase ^ (32u * (o / NHV));
+                static_for<NSUB>([&](auto sub_c) {
+                    constexpr int sub = decltype(sub_c)::value;
+                    lds_read_tr<256 * (o % NHV) + sub * 16 * ROWB>(vb2[b & 1][NSUB * j + sub], vx);
+                });
+            });
+        };
+        rdv(std::integral_constant<int, 0>{});
+        static_for<NPB>([&](auto b_c) {
+            constexpr int b = decltype(b_c)::value;
+            u32x2 (&cur)[NSUB * PB] = vb2[b & 1];
+            if constexpr (b + 1 < NPB) rdv(std::integral_constant<int, b + 1>{});
+            lds_wait<(b + 1 < NPB) ? NSUB * PB : 0>(cur);
+            if constexpr (NSUB == 2) {
 #pragma unroll
                 for (int j = 0; j < PB; j++)
-                    asm volatile("ds_read_b64_tr_b16 %0, %1" : "=v"(dst[j]) : "v"((vbase + sub * 16 * ROWB) ^ (32u * (d0 + j))) : "memory");
-            };
-            rdv(0, vb2[0]);
 #pragma unroll
-            for (int b = 0; b < NPB; b++) {
-                u32x2 (&cur)[PB] = vb2[b & 1];
-                if (b + 1 < NPB) {
-                    rdv(b + 1, vb2[(b + 1) & 1]);
-                    asm volatile("s_waitcnt lgkmcnt(4)" : "+v"(cur[0]), "+v"(cur[1]), "+v"(cur[2]), "+v"(cur[3])::"memory");
-                } else {
-                    asm volatile("s_waitcnt lgkmcnt(0)" : "+v"(cur[0]), "+v"(cur[1]), "+v"(cur[2]), "+v"(cur[3])::"memory");
+                    for (int rb = 0; rb < RB; rb++) {
+                        f32x4 &c = acc[rb][db_of(b * PB + j)];
+                        c = mfma_pv32_hi<F16>(u32x4{cur[2 * j][0], cur[2 * j][1], cur[2 * j + 1][0], cur[2 * j + 1][1]},
+                                              pop[0][rb], pop[1][rb], c);
+                    }
+#pragma unroll
+                for (int j = 0; j < PB; j++)
+#pragma unroll
+                    for (int rb = 0; rb < RB; rb++) {
+                        f32x4 &c = acc[rb][db_of(b * PB + j)];
+                        c = mfma_pv32_lo<F16>(u32x4{cur[2 * j][0], cur[2 * j][1], cur[2 * j + 1][0], cur[2 * j + 1][1]},
+                                              pop[0][rb], pop[1][rb], c);
+                    }
+            } else {
+#pragma unroll
+                for (int j = 0; j < PB; j++) {
+                    f32x4 &c = acc[0][db_of(b * PB + j)];
+                    c = mfma_pv16<F16, KVT != DT_FP32>(cur[j], pop[0][0], c);
                 }
-                const int sub = b / (DB / PB), d0 = (b % (DB / PB)) * PB;
-#pragma unroll
-                for (int j = 0; j < PB; j++) acc[0][d0 + j] = mfma_pv16<F16, KVT != DT_FP32>(cur[j], pop[sub][0], acc[0][d0 + j]);
-                if (pt < NPART && b % 4 == 3) issue_pt(nxt, pt++);
             }
-        }
-        while (pt < NPART) issue_pt(nxt, pt++);
+            if (b == 0 || b == NPB / 2) issue_pt(nxt, pt++);
+        });
     };
 
     // The wave's keys of step it start at jw(it) = (s0 + it) * SK + kg * KT. It attends steps [it0, it1]: before
@@ -474,22 +520,17 @@ prefill_kernel(const PrefArgs a) {
     const int it0 = __builtin_amdgcn_readfirstlane(max(0, -fdiv(-(wlo_all - Cf::KT + 1 - jb), SK)));
     const int it1 = __builtin_amdgcn_readfirstlane(whi_all < 0 ? -1 : min(nsteps - 1, fdiv(whi_all - jb, SK)));
     auto sync_step = [&](int it) {
-        // Step it is the oldest load batch in flight; up to NS-2 younger steps may stay in flight.
-        wait_steps<DMA ? 2 * NLD : 0>(min(NS - 2, nsteps - 1 - it));
-        __syncthreads();                                                // everyone's step it, and step it-1 is consumed
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");                // this wave's loads of step it have landed
+        __syncthreads();                                                // everyone's have, and step it-1 is consumed
         it_cur = it;
-        return it + NS - 1 < nsteps ? it + NS - 1 : -1;
+        return it + 1 < nsteps ? it + 1 : -1;
     };
     int it = 0;
     for (; it < min(it0, nsteps); it++) issue(sync_step(it));
     for (; it <= it1; it++) {
-        const int nxt = sync_step(it);
-        const int jw = (s0 + it) * SK + kg * Cf::KT;
-        const unsigned stage = (it % NS) * Cf::STAGE;
-        int act = 0;                                                    // wave-uniform mask of active row blocks
-#pragma unroll
-        for (int rb = 0; rb < RB; rb++) act |= (jw > whi[rb] || jw + Cf::KT - 1 < wlo[rb]) ? 0 : 1 << rb;
-        step(RB == 1 ? 1 : __builtin_amdgcn_readfirstlane(act), jw, stage, prep(nxt));
+        const StepLd nxt = prep(sync_step(it));
+        qk_softmax(it, nxt);
+        pv(it, nxt);
     }
     for (; it < nsteps; it++) issue(sync_step(it));
     // The no-op loads of the last steps still write (zeros) into a stage: drain them before the merge reuses the
@@ -511,7 +552,10 @@ prefill_kernel(const PrefArgs a) {
     }
     __syncthreads();
     float *xb = reinterpret_cast<float *>(smem);                        // exchange (reuses the tiles)
-    auto slot = [](int sender, int owner) { return sender < owner ? sender : sender - 1; };
+    auto xslot = [&](int rb, int owner, int sender) {
+        return xb + ((((size_t)(rb * RG + rg) * KG + owner) * (KG - 1) + (sender < owner ? sender : sender - 1)) * 16 + ln) * Cf::XSTR + 4 * g;
+    };
+    float f[RB];
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
         const int srow = rb * 16 + ln;
@@ -524,12 +568,11 @@ prefill_kernel(const PrefArgs a) {
             const float mk = stm[(rg * KG + k) * RB * 16 + srow];
             if (mk != kNegInf) L += stl[(rg * KG + k) * RB * 16 + srow] * fast_exp2(mk - M);
         }
-        float f = (m[rb] == kNegInf) ? 0.f : fast_exp2(m[rb] - M);
-        if (a.kv_split <= 0) f *= (L > 0.f ? 1.f / L : 0.f);
+        f[rb] = (m[rb] == kNegInf) ? 0.f : fast_exp2(m[rb] - M);
+        if (a.kv_split <= 0) f[rb] *= (L > 0.f ? 1.f / L : 0.f);
         const int rho = lrow[rb] + ln;
-        const bool rvalid = rho < hrows[rb];
-        const int r = seq * p.T + htok[rb] + (rvalid ? rho / GRP : 0), h = kvh * GRP + (rvalid ? rho % GRP : 0);
-        if (kg == 0 && g == 0 && rvalid) {
+        if (kg == 0 && g == 0 && rho < hrows) {
+            const int t = tok_of(rho), r = seq * p.T + htok + t, h = kvh * GRP + rho - t * GRP;
             if (a.kv_split > 0) {
                 const size_t pi = ((size_t)r * NQ + h) * a.part.ns_cap + sp;
                 a.part.m[pi] = M; a.part.l[pi] = L;
@@ -541,68 +584,66 @@ prefill_kernel(const PrefArgs a) {
         static_for<KG>([&](auto o_c) {
             constexpr int O = decltype(o_c)::value;
             if (O == kg) return;
-            float *dst = xb + ((((size_t)rg * KG + O) * (KG - 1) + slot(kg, O)) * 16 + ln) * Cf::XSTR + 4 * g;
+            float *dst = xslot(rb, O, kg);
 #pragma unroll
-            for (int j = 0; j < DO; j++) *reinterpret_cast<f32x4 *>(dst + 16 * j) = acc[rb][O * DO + j] * f;
+            for (int j = 0; j < DO; j++) *reinterpret_cast<f32x4 *>(dst + 16 * j) = acc[rb][O * DO + j] * f[rb];
         });
-        __syncthreads();
+    }
+    __syncthreads();
+#pragma unroll
+    for (int rb = 0; rb < RB; rb++) {
+        const int rho = lrow[rb] + ln;
+        if (rho >= hrows) continue;
+        const int t = tok_of(rho);
+        const size_t ro = (size_t)(seq * p.T + htok + t) * NQ + kvh * GRP + rho - t * GRP;     // output row
         static_for<KG>([&](auto o_c) {
             constexpr int O = decltype(o_c)::value;
-            if (O != kg || !rvalid) return;
+            if (O != kg) return;
 #pragma unroll
             for (int j = 0; j < DO; j++) {
                 f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int k = 0; k < KG; k++) {
-                    if (k == O) o = (k == 0) ? acc[rb][O * DO + j] * f : o + acc[rb][O * DO + j] * f;
-                    else {
-                        const f32x4 x = *reinterpret_cast<const f32x4 *>(
-                            xb + ((((size_t)rg * KG + O) * (KG - 1) + slot(k, O)) * 16 + ln) * Cf::XSTR + 4 * g + 16 * j);
-                        o = (k == 0) ? x : o + x;
-                    }
+                    const f32x4 x = k == O ? acc[rb][O * DO + j] * f[rb] : *reinterpret_cast<const f32x4 *>(xslot(rb, O, k) + 16 * j);
+                    o = k == 0 ? x : o + x;
                 }
                 const int d = 16 * (O * DO + j) + 4 * g;
                 if (a.kv_split > 0) {
-                    const size_t pi = ((size_t)r * NQ + h) * a.part.ns_cap + sp;
-                    *reinterpret_cast<f32x4 *>(a.part.acc + pi * HD + d) = o;
-                    continue;
-                }
-                const size_t ob = ((size_t)r * NQ + h) * HD + d;
-                if constexpr (OT == DT_FP32) *reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(p.O) + ob) = o;
-                else {
+                    *reinterpret_cast<f32x4 *>(a.part.acc + (ro * a.part.ns_cap + sp) * HD + d) = o;
+                } else if constexpr (OT == DT_FP32) {
+                    *reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(p.O) + ro * HD + d) = o;
+                } else {
                     const u32x2 wv = u32x2{pack2<OT == DT_F16>(o.x, o.y), pack2<OT == DT_F16>(o.z, o.w)};
-                    *reinterpret_cast<u32x2 *>(reinterpret_cast<uint16_t *>(p.O) + ob) = wv;
+                    *reinterpret_cast<u32x2 *>(reinterpret_cast<uint16_t *>(p.O) + ro * HD + d) = wv;
                 }
             }
         });
-        if (rb + 1 < RB) __syncthreads();                               // the next block reuses the exchange
     }
 }
 
 // ---------------------------------------------------------------- host side
-// Tile shapes. HD 128/256: 8 waves (two per SIMD, so one wave's MFMAs overlap the other's softmax and LDS
-// traffic) as 4 row groups x 2 key groups, 16 rows and HD accumulator columns per wave, a 64-row workgroup tile
-// (two 32-row half tiles), 64-key steps (two 16-key sub-tiles per wave) in two LDS stages. HD 512: the same 8 waves
-// and 64-row tile with 32-key steps (a 32-key stage of HD 512 is 64 KB) and 252 VGPRs (a 16 x 512 accumulator per
-// wave); the 4-wave 32-row tile it replaces ran the Gemma4 global prompt (T = 1024, one KV head, 16 q-heads) in
-// two rounds of 256 workgroups: 92 vs 55 us.
-// Measured alternatives at HD 256 (config 3, T = 1024): 4 waves over a 32-row tile, two workgroups per CU, 38.8
-// vs 30.0 us; 16-key steps per wave, 33.1 us; two 16-row blocks per wave (one wave per SIMD), 36.9 us.
-// HD 256, wide tile (W = 1): 12 waves (6 row groups, three per SIMD, 168 VGPRs) over a 96-row tile. Its half tile
-// of 48 rows holds 8 tokens of a 6-head GQA group where the 32-row one holds 5 (30 rows), so the Qwen3.5 prompt
-// (T = 1024, 24 q-heads over 4 KV heads) is 256 workgroups, one round, instead of 412 in two: 53.4 vs 37.2 us. It
-// runs a prompt only when it needs fewer rounds of resident workgroups than the 64-row tile (config 3 is one
-// round either way, and 31.0 vs 35.5 us there). The two tiles share the step (64 keys), the key groups and the
-// merge order, so a row's bits do not depend on which one ran it.
-// WPE: waves per SIMD the register allocation must allow. PAIR: whether a workgroup may take the causal
-// half-tile pair (i, n-1-i) (one workgroup per CU) instead of neighbours.
+// Tile shapes: 8 waves (two per SIMD) as 4 row groups x 2 key groups, 16 rows and HD accumulator columns per wave, a
+// 64-row workgroup tile, 64-key steps (two 16-key sub-tiles per wave) in two LDS stages. HD 512: 32-key steps (a 32-key
+// stage of HD 512 is 64 KB) and a 16 x 512 accumulator per wave.
+// HD 256 has two larger tiles for launches of more than one round of 64-row workgroups; all three share the step, the
+// key groups and the merge order, so a row's bits do not depend on which one ran it.
+//   W = 1: 12 waves (6 row groups, three per SIMD, 164 VGPRs), 96 rows.
+//   W = 2: 8 waves of two 16-row blocks each (256 VGPRs), 128 rows: every K and V fragment read from LDS feeds two MFMAs,
+//          so a row costs 18 ns per 64-key step against 22 ns at 64 rows (bf16).
+// What bounds a step: MFMA issue and VALU issue add up on a SIMD (a probe with two waves per SIMD measures 16.5 cycles per
+// 16x16x32 MFMA and about 2.2 more for every VALU op beside it), and a 128-row bf16 step holds 192 MFMAs (3170 cycles)
+// and about 380 VALU ops per SIMD; it runs in about 5000 cycles. Neither the LDS (256 bytes per clock against 320 KB per
+// step) nor the L2 stream (without the loads the 4096-token window prompt gains 3%) is near its limit, and letting the
+// second wave of each SIMD run half a step behind the first, to put one's MFMAs under the other's softmax, changed nothing.
+// WPE: waves per SIMD the register allocation must allow.
 template <int HD, int W> struct PrefTile;
-template <> struct PrefTile<128, 0> { static constexpr int RB = 1, RG = 4, KG = 2, NS = 2, NSUB = 2, WPE = 2; static constexpr bool PAIR = true; };
-template <> struct PrefTile<256, 0> { static constexpr int RB = 1, RG = 4, KG = 2, NS = 2, NSUB = 2, WPE = 2; static constexpr bool PAIR = true; };
-template <> struct PrefTile<256, 1> { static constexpr int RB = 1, RG = 6, KG = 2, NS = 2, NSUB = 2, WPE = 3; static constexpr bool PAIR = true; };
-template <> struct PrefTile<512, 0> { static constexpr int RB = 1, RG = 4, KG = 2, NS = 2, NSUB = 1, WPE = 2; static constexpr bool PAIR = true; };
+template <> struct PrefTile<128, 0> { static constexpr int RB = 1, RG = 4, KG = 2, NSUB = 2, WPE = 2; };
+template <> struct PrefTile<256, 0> { static constexpr int RB = 1, RG = 4, KG = 2, NSUB = 2, WPE = 2; };
+template <> struct PrefTile<256, 1> { static constexpr int RB = 1, RG = 6, KG = 2, NSUB = 2, WPE = 3; };
+template <> struct PrefTile<256, 2> { static constexpr int RB = 2, RG = 4, KG = 2, NSUB = 2, WPE = 2; };
+template <> struct PrefTile<512, 0> { static constexpr int RB = 1, RG = 4, KG = 2, NSUB = 1, WPE = 2; };
 template <int HD, int W>
-using PrefTileCfg = PrefCfg<HD, PrefTile<HD, W>::RB, PrefTile<HD, W>::RG, PrefTile<HD, W>::KG, PrefTile<HD, W>::NS,
+using PrefTileCfg = PrefCfg<HD, PrefTile<HD, W>::RB, PrefTile<HD, W>::RG, PrefTile<HD, W>::KG,
                             PrefTile<HD, W>::NSUB>;
 
 template <int HD, int W, int KVT, int QT, int OT>
@@ -610,7 +651,7 @@ static hipError_t launch_pref_t(const PrefArgs &a, dim3 grid, hipStream_t st) {
     using T = PrefTile<HD, W>;
     using Cf = PrefTileCfg<HD, W>;
     static bool configured = false;
-    auto kern = prefill_kernel<HD, T::RB, T::RG, T::KG, T::NS, T::NSUB, T::WPE, KVT, QT, OT>;
+    auto kern = prefill_kernel<HD, T::RB, T::RG, T::KG, T::NSUB, T::WPE, KVT, QT, OT>;
     if (!configured) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)Cf::LDS);
@@ -625,32 +666,38 @@ template <int KVT, int QT, int OT>
 static hipError_t pref_dispatch_hd(const PrefArgs &a, int wide, dim3 grid, hipStream_t st) {
     switch (a.p.HD) {
     case 128: return launch_pref_t<128, 0, KVT, QT, OT>(a, grid, st);
-    case 256: return wide ? launch_pref_t<256, 1, KVT, QT, OT>(a, grid, st) : launch_pref_t<256, 0, KVT, QT, OT>(a, grid, st);
+    case 256:
+        if constexpr (KVT != DT_FP32) {
+            if (wide == 1) return launch_pref_t<256, 1, KVT, QT, OT>(a, grid, st);
+            if (wide == 2) return launch_pref_t<256, 2, KVT, QT, OT>(a, grid, st);
+        }
+        return launch_pref_t<256, 0, KVT, QT, OT>(a, grid, st);
     case 512: return launch_pref_t<512, 0, KVT, QT, OT>(a, grid, st);
     default: return hipErrorInvalidValue;
     }
 }
 
-// Per tile shape (head dim, W): rows of a half tile, workgroups resident per CU, and whether it takes causal
-// half-tile pairs. HD 128 and 512 have the one shape.
-struct PrefShape { int hr, per_cu; bool pair; };
-template <int HD, int W> static PrefShape pref_shape_t() {
-    return PrefShape{PrefTileCfg<HD, W>::HR, (int)std::max<size_t>(1, (160u << 10) / PrefTileCfg<HD, W>::LDS),
-                     PrefTile<HD, W>::PAIR};
+// Per tile shape (head dim, W): rows of a half tile, workgroups resident per CU, keys per step, and the measured cost of
+// a workgroup on bf16 caches in us: its start and end, a step with both half tiles at work, and a step with one.
+struct PrefShape { int hr, per_cu, sk; float ov, full, half; };
+template <int HD, int W> static PrefShape pref_shape_t(float ov, float full, float half) {
+    using Cf = PrefTileCfg<HD, W>;
+    return PrefShape{Cf::HR, (int)std::max<size_t>(1, (160u << 10) / Cf::LDS), Cf::SK, ov, full, half};
 }
 static PrefShape pref_shape(int HD, int wide) {
     switch (HD) {
-    case 128: return pref_shape_t<128, 0>();
-    case 256: return wide ? pref_shape_t<256, 1>() : pref_shape_t<256, 0>();
-    case 512: return pref_shape_t<512, 0>();
-    default: return PrefShape{0, 1, false};
+    case 128: return pref_shape_t<128, 0>(4.5f, 0.8f, 0.6f);
+    case 256:
+        return wide == 2 ? pref_shape_t<256, 2>(9.f, 2.35f, 1.43f)
+               : wide    ? pref_shape_t<256, 1>(7.f, 1.9f, 1.25f)
+                         : pref_shape_t<256, 0>(5.5f, 1.45f, 1.05f);
+    case 512: return pref_shape_t<512, 0>(8.f, 1.37f, 1.08f);
+    default: return PrefShape{0, 1, 64, 0.f, 0.f, 0.f};
     }
 }
 static int pref_half_rows(int HD) { return pref_shape(HD, 0).hr; }
 static int pref_per_cu(int HD) { return pref_shape(HD, 0).per_cu; }
 
-// Key split for kv_split = -1: when the unsplit grid would fill at most half of the workgroup slots (a short run
-// of queries over a long cached prefix), cut the keys into as many absolute splits as whole grids fit on them.
 size_t prefill_lds_bytes(int HD) {
     switch (HD) {
     case 128: return PrefTileCfg<128, 0>::LDS;
@@ -660,22 +707,98 @@ size_t prefill_lds_bytes(int HD) {
     }
 }
 
+// CUs of the current device (0: unknown).
+static int device_cus() {
+    static std::atomic<int> cus[64];
+    int dev = 0;
+    if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
+    int n = cus[dev].load(std::memory_order_relaxed);
+    if (n == 0 && hipDeviceGetAttribute(&n, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess)
+        cus[dev].store(n, std::memory_order_relaxed);
+    return n;
+}
+
+// Key split for kv_split = -1: when the unsplit grid would fill at most half of the workgroup slots (a short run
+// of queries over a long cached prefix), cut the keys into as many absolute splits as whole grids fit on them.
 int prefill_auto_split(const Problem &p) {
     if (p.NQ % p.NKV) return 0;
     const int GRP = p.NQ / p.NKV, HR = pref_half_rows(p.HD);
     if (HR == 0 || GRP > HR) return 0;
     const int tqh = HR / GRP, nht = (p.T + tqh - 1) / tqh;
     const long nwg = (long)p.nseq * p.NKV * ((nht + 1) / 2);
-    int dev = 0, ncu = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        return 0;
-    const long slots = (long)ncu * pref_per_cu(p.HD);
+    const long slots = (long)device_cus() * pref_per_cu(p.HD);
     if (nwg <= 0 || 2 * nwg > slots) return 0;
     const int nsplit = (int)(slots / nwg);
     const int keys = p.max_pos + 1;
     int ks = (keys + nsplit - 1) / nsplit;
     ks = ((ks + 63) / 64) * 64;
     return ks >= keys ? 0 : ks;
+}
+
+// How a launch is cut into work items: the tile shape, and one tile per item (a full one or, `one_half`, a half tile whose
+// other waves only load) or a causal pair of half tiles.
+struct PrefPlan { int wide, pair, tqh, nht; };
+static PrefPlan pref_plan(const PrefShape &sh, int wide, int GRP, int T, bool pair, bool one_half) {
+    const int tqh = (pair || one_half ? 1 : 2) * sh.hr / GRP;
+    return PrefPlan{wide, pair ? 1 : 0, tqh, (T + tqh - 1) / tqh};
+}
+// Estimated time of a plan in us: the items, longest first, dealt in a snake over the slots (slot c takes items c, 2K-1-c,
+// 2K+c, ...), which is about what longest-first dispatch gives; the longest of five slots counts.
+static float pref_cost(const PrefShape &sh, const PrefPlan &pl, const Problem &p, int kv_split, int nsplit, int slots) {
+    const int heads = p.nseq * p.NKV, base = std::max(0, p.max_pos - p.T + 1), GRP = p.NQ / p.NKV;
+    const bool both = pl.pair || pl.tqh * GRP > sh.hr;
+    auto cost = [&](long i) {
+        const int r = (int)(i / heads / nsplit), t0 = (pl.nht - 1 - r) * pl.tqh, hi = base + std::min(p.T, t0 + pl.tqh);
+        const int lo = p.window > 0 ? std::max(0, base + t0 - p.window + 1) : 0;
+        int n = (hi - 1) / sh.sk - lo / sh.sk + 1;
+        if (kv_split > 0) n = std::min(n, kv_split / sh.sk);
+        if (!pl.pair) return sh.ov + n * (both ? sh.full : sh.half);
+        const int s = std::min(n, r == pl.nht - 1 - r ? 0 : (base + (r + 1) * pl.tqh - 1) / sh.sk + 1);
+        return sh.ov + s * sh.full + (n - s) * sh.half;
+    };
+    const long items = (long)heads * nsplit * (pl.pair ? (pl.nht + 1) / 2 : pl.nht), rounds = (items + slots - 1) / slots;
+    const long every = std::max(1L, rounds / 16);                       // sampled rounds of a long launch
+    float worst = 0.f;
+    for (int k = 0; k < 5; k++) {
+        const long c = (long)(slots - 1) * k / 4;
+        float sum = 0.f;
+        for (long r = 0; r < rounds; r += every) {
+            const long i = r * slots + (r & 1 ? slots - 1 - c : c);
+            if (i < items) sum += cost(i) * (float)std::min(every, rounds - r);
+        }
+        worst = std::max(worst, sum);
+    }
+    return worst;
+}
+// The plan of a launch. If half tiles of the narrow shape fit the device in one round, one each: the longest item then has
+// the cheapest steps (a causal pair would only add the short half's). Otherwise the cheapest by pref_cost among the shapes
+// (the larger ones on 16-bit caches: the fp32 cache's register staging spills in them) with one tile per item or, for
+// causal prompts whose work varies (no window, prefix shorter than the chunk), pairs. Measured at bf16 unless said:
+//   16 q-heads over 8 KV heads, T = 1024: pairs of 32 rows 25.7 us; 64-row tiles 29.6, 96-row pairs 30.7, 128-row pairs 35.1
+//   the same, T = 4096, window 1024: 128-row tiles 101 us; 64-row 114, 96-row 117
+//   24 over 4, T = 1377 (f16): 96-row tiles 42.4 us; 64-row tiles 50.1 and pairs 64.6, 128-row tiles 50.5, 96-row pairs 54.7
+//   16 over 1 of 512, T = 1024: pairs 46.1 us, 64-row tiles 55.0
+static PrefPlan choose_plan(const Problem &p, int kv_split, int nsplit, int ncu) {
+    const int GRP = p.NQ / p.NKV;
+    const PrefShape s0 = pref_shape(p.HD, 0);
+    const PrefPlan small = pref_plan(s0, 0, GRP, p.T, false, true);
+    const int slots0 = std::max(ncu, 1) * s0.per_cu;
+    if ((long)p.nseq * p.NKV * nsplit * small.nht <= slots0) return small;
+    const bool causal = kv_split == 0 && p.window == 0 && p.max_pos < 2 * p.T;
+    PrefPlan best = pref_plan(s0, 0, GRP, p.T, causal, false);
+    float cost = pref_cost(s0, best, p, kv_split, nsplit, slots0);
+    auto consider = [&](const PrefShape &sh, const PrefPlan &pl) {
+        const float c = pref_cost(sh, pl, p, kv_split, nsplit, std::max(ncu, 1) * sh.per_cu);
+        if (c < cost) { cost = c; best = pl; }
+    };
+    if (causal) consider(s0, pref_plan(s0, 0, GRP, p.T, false, false));
+    if (p.HD == 256 && p.kv_dtype != DT_FP32)
+        for (int w = 1; w <= 2; w++) {
+            const PrefShape sh = pref_shape(256, w);
+            consider(sh, pref_plan(sh, w, GRP, p.T, false, false));
+            if (causal) consider(sh, pref_plan(sh, w, GRP, p.T, true, false));
+        }
+    return best;
 }
 
 hipError_t launch_prefill(const Problem &p, int kv_split, const Partials &part, hipStream_t st) {
@@ -685,30 +808,17 @@ hipError_t launch_prefill(const Problem &p, int kv_split, const Partials &part, 
     if (kv_split < 0 || (kv_split > 0 && kv_split % 64)) return hipErrorInvalidValue;
     const int nsplit = kv_split > 0 ? p.max_pos / kv_split + 1 : 1;
     if (kv_split > 0 && nsplit > part.ns_cap) return hipErrorInvalidValue;
-    int dev = 0, ncu = 0;
-    if (hipGetDevice(&dev) != hipSuccess || hipDeviceGetAttribute(&ncu, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess)
-        ncu = 0;
-    // Workgroups of a tile shape: half tiles of tqh tokens, two per workgroup.
-    auto wgs = [&](const PrefShape &sh) { return (long)p.nseq * p.NKV * (((p.T + sh.hr / GRP - 1) / (sh.hr / GRP) + 1) / 2); };
-    auto rounds = [&](const PrefShape &sh) { const long slots = (long)std::max(ncu, 1) * sh.per_cu; return (wgs(sh) + slots - 1) / slots; };
-    // The wide HD 256 tile, when it takes fewer rounds of resident workgroups (unsplit prompts, 16-bit caches: the
-    // fp32 cache's register staging spills in it).
-    int wide = 0;
-    if (p.HD == 256 && kv_split == 0 && p.kv_dtype != DT_FP32 && ncu > 0 && GRP <= pref_shape(256, 1).hr &&
-        rounds(pref_shape(256, 1)) < rounds(pref_shape(256, 0)))
-        wide = 1;
-    const PrefShape sh = pref_shape(p.HD, wide);
-    const int tqh = sh.hr / GRP;
-    const int nht = (p.T + tqh - 1) / tqh;
-    // Pair half tiles (i, n-1-i) when causal work varies across the prompt (no window, prefix shorter than the
-    // chunk); otherwise a workgroup takes two neighbouring half tiles.
-    const int pair = (sh.pair && kv_split == 0 && p.window == 0 && nht >= 2 && p.max_pos < 2 * p.T) ? 1 : 0;
-    const int nitems = ((nht + 1) / 2) * nsplit;
-    const long nwg = (long)p.nseq * p.NKV * nitems;
+    const int ncu = device_cus();
+    const PrefPlan pl = choose_plan(p, kv_split, nsplit, ncu);
+    const int wide = pl.wide, per_cu = pref_shape(p.HD, wide).per_cu, heads = p.nseq * p.NKV;
+    const long nitems = (long)(pl.pair ? (pl.nht + 1) / 2 : pl.nht) * nsplit, nwg = heads * nitems;
     if (nwg <= 0 || nwg > (1L << 30)) return hipErrorInvalidConfiguration;
-    const int fold = (sh.per_cu >= 2 && nwg <= (long)sh.per_cu * ncu) ? 1 : 0;
-    PrefArgs a{p, part, kv_split, nht, nsplit, tqh, pair, nitems, (int)nwg, p.scale * kLog2e, fold};
-    dim3 grid((unsigned)(8 * ((nwg + 7) / 8)));
+    const int fold = (per_cu >= 2 && nwg <= (long)per_cu * ncu) ? 1 : 0;
+    const int ways = heads < 8 && 8 % heads == 0 ? 8 / heads : heads % 8 == 0 ? -(heads / 8) : 0;
+    const long per = ways > 0 ? (nitems + ways - 1) / ways : (nwg + 7) / 8;
+    PrefArgs a{p, part, kv_split, pl.nht, nsplit, pl.tqh, pl.pair, (int)nitems, heads, GRP, p.scale * kLog2e, fold,
+               (reinterpret_cast<uintptr_t>(p.Q) & 15) == 0 ? 1 : 0, 65535 / GRP + 1, ways};
+    dim3 grid((unsigned)(8 * per));
     hipError_t e = hipErrorInvalidValue;
     const int kv = p.kv_dtype, q = p.q_dtype, o = p.o_dtype;
     if (kv == DT_F16 && q == DT_FP32 && o == DT_FP32) e = pref_dispatch_hd<DT_F16, DT_FP32, DT_FP32>(a, wide, grid, st);
