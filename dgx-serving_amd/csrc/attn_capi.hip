@@ -296,7 +296,7 @@ hipError_t timed_launch(hipStream_t st, F &&launch) {
     return e;
 }
 
-// How verify_kernel cuts its runs (dgx_attn_verify_runs): 0 = each sequence's absolute key chunks, 1 = equal runs
+// How batched verify divides the keys (dgx_attn_verify_runs): 0 = each sequence's absolute key chunks, 1 = equal runs
 // over the whole batch.
 std::atomic<int> g_verify_runs{0};
 

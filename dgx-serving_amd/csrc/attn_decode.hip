@@ -29,6 +29,7 @@ struct DecodeArgs {
     Problem p;
     Partials part;
     int C;
+    uint32_t Cm;       // div_magic(C)
     float sl2;
 };
 
@@ -49,62 +50,6 @@ struct DecodeCfg {
 };
 
 
-// Work item blockIdx.x -> (sequence, chunk c, kv head blockIdx.x % NKV), enumerating only the chunks that hold keys
-// of the sequence's tokens (kv head fastest): the workgroups with work come first in launch order and the dispatcher
-// spreads them over all CUs; the tail of the upper-bound grid (false) exits at once. Two phases: first every chunk
-// of each sequence but one, then that one: the shorter of its first and last chunk (both partial under a sliding
-// window, only the last otherwise). The dispatcher hands workgroups out in
-// index order and a CU that receives more workgroups than the others shares its bandwidth among them, so the short
-// items go last, where they land on the CUs that get a third workgroup (measured: a CU with three full items runs
-// 20% longer than one with two).
-__device__ __forceinline__ bool find_item(const Problem &p, int C, int &seq, int &c, int &lo, int &hi) {
-    const int lane_ = threadIdx.x & 63, cmax = p.max_pos / C;
-    int rest = (int)blockIdx.x / p.NKV;
-    seq = -1; c = 0;
-    for (int phase = 0; phase < 2; phase++) {
-        for (int s0 = 0; s0 < p.nseq; s0 += 64) {
-            int n = 0, first = 0, lo_s = INT_MAX, hi_s = 0;   // key range of the sequence's tokens
-            if (s0 + lane_ < p.nseq) {
-                for (int t = 0; t < p.T; t++) {
-                    const int ps = tok_pos(p, s0 + lane_, t);
-                    lo_s = min(lo_s, win_lo(ps, p.window)); hi_s = max(hi_s, ps + 1);
-                }
-                first = lo_s / C;
-                n = max(0, min((hi_s - 1) / C, cmax) - first + 1);
-            }
-            const int m = phase == 0 ? max(n - 1, 0) : min(n, 1);   // items of this sequence in this phase
-            // The phase-1 chunk: the shorter of the first and the last chunk (a sliding window's first chunk is
-            // partial too); phase 0 takes the others in order.
-            int sh = 0;
-            if (n >= 2) {
-                const int kf = min(hi_s, (first + 1) * C) - lo_s, kl = hi_s - max(lo_s, (first + n - 1) * C);
-                sh = kf < kl ? 0 : n - 1;
-            }
-            int incl = m;                                  // inclusive prefix sum over the 64 lanes
-#pragma unroll
-            for (int o = 1; o < 64; o <<= 1) {
-                const int y = __shfl_up(incl, o);
-                if (lane_ >= o) incl += y;
-            }
-            const unsigned long long hit = __ballot(incl > rest);
-            if (hit) {
-                const int l = __builtin_ctzll(hit);
-                seq = s0 + l;
-                if (phase == 0) {
-                    const int r = rest - (__shfl(incl, l) - __shfl(m, l));
-                    c = __shfl(first, l) + (r < __shfl(sh, l) ? r : r + 1);
-                } else {
-                    c = __shfl(first, l) + __shfl(sh, l);
-                }
-                lo = __shfl(lo_s, l); hi = __shfl(hi_s, l);
-                return true;
-            }
-            rest -= __shfl(incl, 63);
-        }
-    }
-    return false;
-}
-
 template <int HD, int NKL_, int RW_, int KVT, int QT, bool EARLY>
 __global__ void __launch_bounds__(NKL_ * RW_ * 64) decode_stream_kernel(const DecodeArgs a) {
     using Cf = DecodeCfg<HD, NKL_, RW_>;
@@ -117,7 +62,7 @@ __global__ void __launch_bounds__(NKL_ * RW_ * 64) decode_stream_kernel(const De
     const Problem &p = a.p;
     const int C = a.C;
     int seq, c, lo, hi;
-    if (!find_item(p, C, seq, c, lo, hi)) return;
+    if (!find_item(p, C, a.Cm, (int)blockIdx.x / p.NKV, seq, c, lo, hi)) return;
     seq = __builtin_amdgcn_readfirstlane(seq); c = __builtin_amdgcn_readfirstlane(c);
     lo = __builtin_amdgcn_readfirstlane(lo); hi = __builtin_amdgcn_readfirstlane(hi);
     const int kvh = (int)blockIdx.x % p.NKV;
@@ -356,18 +301,6 @@ static hipError_t dec_dispatch_hd(const DecodeArgs &a, dim3 grid, int rw, hipStr
     }
 }
 
-// Upper bound of the work items (sequence, chunk, kv head) of a launch: every chunk up to max_pos, or, under a sliding
-// window with consecutive token positions, the at most (window + T - 2) / chunk + 2 chunks a window of window + T - 1
-// keys meets (a 32K-key cache with a 1K window then launches 6 items per sequence and head, not 128).
-static long long decode_items_bound(const Problem &p, int chunk) {
-    long long per = p.max_pos / chunk + 1;
-    if (p.window > 0 && (p.T == 1 || p.pos_mode == 1)) {
-        const long long w = ((long long)p.window + p.T - 2) / chunk + 2;
-        if (w < per) per = w;
-    }
-    return per * p.NKV * p.nseq;
-}
-
 bool decode_stream_supported(const Problem &p) {
     // One 16-row block (RW = 1). The kernel also runs RW = 2..4 row blocks, one wave each per key lane, but then
     // the row waves re-read every tile, which measured slower than the cooperative split kernel on the B=16 x
@@ -380,8 +313,8 @@ hipError_t launch_decode_stream(const Problem &p, int chunk, const Partials &par
     if (!decode_stream_supported(p)) return hipErrorNotSupported;
     if (chunk <= 0 || chunk % 16) return hipErrorInvalidValue;
     if (p.max_pos / chunk + 1 > part.ns_cap) return hipErrorInvalidValue;
-    DecodeArgs a{p, part, chunk, p.scale * kLog2e};
-    const long long items = decode_items_bound(p, chunk);
+    DecodeArgs a{p, part, chunk, div_magic(chunk), p.scale * kLog2e};
+    const long long items = chunk_items_bound(p, chunk) * p.NKV;
     if (items > INT_MAX) return hipErrorInvalidConfiguration;
     dim3 grid((unsigned)items);
     const int rw = (p.T * (p.NQ / p.NKV) + 15) / 16;   // 16-row blocks, one wave each per key lane
@@ -427,7 +360,7 @@ __global__ void __launch_bounds__(128) decode_f32_kernel(const DecodeArgs a) {
     const Problem &p = a.p;
     const int C = a.C;
     int seq, c, lo, hi;
-    if (!find_item(p, C, seq, c, lo, hi)) return;
+    if (!find_item(p, C, a.Cm, (int)blockIdx.x / p.NKV, seq, c, lo, hi)) return;
     seq = __builtin_amdgcn_readfirstlane(seq); c = __builtin_amdgcn_readfirstlane(c);
     lo = __builtin_amdgcn_readfirstlane(lo); hi = __builtin_amdgcn_readfirstlane(hi);
     const int kvh = (int)blockIdx.x % p.NKV;
@@ -591,8 +524,8 @@ hipError_t launch_decode_f32(const Problem &p, int chunk, const Partials &part, 
     if (!decode_f32_supported(p)) return hipErrorNotSupported;
     if (chunk <= 0 || chunk % 16) return hipErrorInvalidValue;
     if (p.max_pos / chunk + 1 > part.ns_cap) return hipErrorInvalidValue;
-    DecodeArgs a{p, part, chunk, p.scale * kLog2e};
-    const long long items = decode_items_bound(p, chunk);
+    DecodeArgs a{p, part, chunk, div_magic(chunk), p.scale * kLog2e};
+    const long long items = chunk_items_bound(p, chunk) * p.NKV;
     if (items > INT_MAX) return hipErrorInvalidConfiguration;
     dim3 grid((unsigned)items);
     if (p.HD == 128) {

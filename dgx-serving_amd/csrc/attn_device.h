@@ -210,9 +210,10 @@ __device__ __forceinline__ __amdgpu_buffer_rsrc_t make_rsrc(const void *base, ui
                                              __builtin_amdgcn_readfirstlane((int)bytes), 0x00020000);
 }
 // 16 bytes per lane from buffer offset voffset into LDS at lds + 16 * lane (gfx950 buffer_load_dwordx4 ... lds).
+template <bool NT = false>   // NT: non-temporal, for data read once
 __device__ __forceinline__ void buffer_load_lds16(__amdgpu_buffer_rsrc_t rsrc, void *lds, int voffset) {
     __builtin_amdgcn_raw_ptr_buffer_load_lds(rsrc, (__attribute__((address_space(3))) void *)(reinterpret_cast<uintptr_t>(lds)),
-                                             16, voffset, 0, 0, 0);
+                                             16, voffset, 0, 0, NT ? 2 : 0);
 }
 
 // Online-softmax rescale threshold (log2 units): the running reference max of a row moves only when a new score

@@ -2,6 +2,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 #include <stdint.h>
+#include <climits>
 
 namespace dgx {
 
@@ -66,9 +67,146 @@ __device__ __forceinline__ int win_lo(int pos, int window) {
     return (window > 0 && pos - window + 1 > 0) ? pos - window + 1 : 0;
 }
 
-// Split-KV decode / verify / tree kernel (waves split the keys of a chunk, small query-row tiles). Verify and tree
-// rows on 16-bit caches at HD <= 256 run verify_kernel: slot_runs cuts its runs at absolute key chunks of each
-// sequence (batch-invariant), otherwise into equal runs over the whole batch (faster, depends on the batch).
+// x / C for 0 <= x < 2^31 and C >= 2, with M = div_magic(C): a runtime division costs a few hundred cycles on the path to a
+// workgroup's first load. x M / 2^32 exceeds x / C by less than a half.
+inline uint32_t div_magic(int C) { return (uint32_t)(0xffffffffu / (uint32_t)C) + 1u; }
+__device__ __forceinline__ int div_by(int x, int C, uint32_t M) {
+    const int q = (int)__umulhi((uint32_t)x, M);
+    return q * C > x ? q - 1 : q;
+}
+
+// Inclusive prefix sum over the 64 lanes on the VALU (DPP row shifts and row broadcasts).
+__device__ __forceinline__ int wave_scan64(int v) {
+    v += __builtin_amdgcn_update_dpp(0, v, 0x111, 0xf, 0xf, false);     // row_shr:1
+    v += __builtin_amdgcn_update_dpp(0, v, 0x112, 0xf, 0xf, false);     // row_shr:2
+    v += __builtin_amdgcn_update_dpp(0, v, 0x114, 0xf, 0xf, false);     // row_shr:4
+    v += __builtin_amdgcn_update_dpp(0, v, 0x118, 0xf, 0xf, false);     // row_shr:8
+    v += __builtin_amdgcn_update_dpp(0, v, 0x142, 0xa, 0xf, false);     // row_bcast:15 into rows 1 and 3
+    v += __builtin_amdgcn_update_dpp(0, v, 0x143, 0xc, 0xf, false);     // row_bcast:31 into rows 2 and 3
+    return v;
+}
+
+// Work item number `rest` -> (sequence, chunk c of C keys) and the key range [lo, hi) of the sequence's tokens,
+// enumerating only the chunks that hold keys of them; called by whole waves with the same `rest`. M = div_magic(C). The
+// workgroups with work come first in launch order and the dispatcher
+// spreads them over all CUs; the tail of the upper-bound grid (false) exits at once. Two phases: first every chunk
+// of each sequence but one, then that one: the shorter of its first and last chunk (both partial under a sliding
+// window, only the last otherwise). The dispatcher hands workgroups out in
+// index order and a CU that receives more workgroups than the others shares its bandwidth among them, so the short
+// items go last, where they land on the CUs that get a third workgroup (measured: a CU with three full items runs
+// 20% longer than one with two).
+// Up to 64 sequences take one position load, one scan and no division; the general form is ~2 us (its scans go through
+// LDS shuffles), which a workgroup spends before its first load.
+__device__ __forceinline__ bool find_item(const Problem &p, int C, uint32_t M, int rest, int &seq, int &c, int &lo, int &hi) {
+    const int lane_ = threadIdx.x & 63, cmax = div_by(p.max_pos, C, M);
+    seq = -1; c = 0;
+    // Key range of sequence s's tokens, its first chunk and chunk count (positions ascend with the token).
+    auto range = [&](int s, int &lo_s, int &hi_s, int &first, int &n) {
+        const int p0 = tok_pos(p, s, 0), p1 = p.T > 1 ? tok_pos(p, s, p.T - 1) : p0;
+        lo_s = win_lo(min(p0, p1), p.window); hi_s = max(p0, p1) + 1;
+        if (p.pos_mode == 0)
+            for (int t = 1; t + 1 < p.T; t++) {             // rows of their own positions
+                const int ps = tok_pos(p, s, t);
+                lo_s = min(lo_s, win_lo(ps, p.window)); hi_s = max(hi_s, ps + 1);
+            }
+        first = div_by(max(lo_s, 0), C, M);
+        n = hi_s > 0 ? max(0, min(div_by(hi_s - 1, C, M), cmax) - first + 1) : 0;
+    };
+    // The phase-1 chunk of a sequence, counted from its first: the shorter of the first and the last.
+    auto short_chunk = [&](int lo_s, int hi_s, int first, int n) {
+        const int kf = min(hi_s, (first + 1) * C) - lo_s, kl = hi_s - max(lo_s, (first + n - 1) * C);
+        return n >= 2 && kf >= kl ? n - 1 : 0;
+    };
+    if (p.nseq <= 64) {
+        int lo_s = 0, hi_s = 0, first = 0, n = 0;
+        if (lane_ < p.nseq) range(lane_, lo_s, hi_s, first, n);
+        const int m = max(n - 1, 0), incl = wave_scan64(m), total = __builtin_amdgcn_readlane(incl, 63);
+        unsigned long long hit;
+        if (rest < total) {
+            hit = __ballot(incl > rest);
+        } else {                                            // the (rest - total)-th sequence with keys
+            const unsigned long long some = __ballot(n > 0);
+            const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(some >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)some, 0));
+            hit = __ballot(n > 0 && rank == rest - total);
+            if (!hit) return false;
+        }
+        const int l = __builtin_ctzll(hit);
+        const int sh = short_chunk(lo_s, hi_s, first, n), r = rest - (incl - m);    // of lane l: its own
+        const int cc = first + (rest >= total ? sh : r < sh ? r : r + 1);
+        seq = l;
+        c = __builtin_amdgcn_readlane(cc, l); lo = __builtin_amdgcn_readlane(lo_s, l); hi = __builtin_amdgcn_readlane(hi_s, l);
+        return true;
+    }
+    for (int phase = 0; phase < 2; phase++) {
+        for (int s0 = 0; s0 < p.nseq; s0 += 64) {
+            int lo_s = 0, hi_s = 0, first = 0, n = 0;
+            if (s0 + lane_ < p.nseq) range(s0 + lane_, lo_s, hi_s, first, n);
+            const int m = phase == 0 ? max(n - 1, 0) : min(n, 1);   // items of this sequence in this phase
+            const int sh = short_chunk(lo_s, hi_s, first, n), incl = wave_scan64(m);
+            const unsigned long long hit = __ballot(incl > rest);
+            if (hit) {
+                const int l = __builtin_ctzll(hit), r = rest - (incl - m);
+                const int cc = first + (phase == 1 ? sh : r < sh ? r : r + 1);
+                seq = s0 + l;
+                c = __builtin_amdgcn_readlane(cc, l); lo = __builtin_amdgcn_readlane(lo_s, l); hi = __builtin_amdgcn_readlane(hi_s, l);
+                return true;
+            }
+            rest -= __builtin_amdgcn_readlane(incl, 63);
+        }
+    }
+    return false;
+}
+
+// Run number `rest` of a launch with room for `slots` runs at once -> the chunks [c0, c1) of sequence seq. While the chunks
+// of all sequences outnumber the slots, a run takes g of them (a sequence's cut evenly), with the smallest g whose runs
+// fit the slots: one round of long runs saves the start of a workgroup per chunk, and each chunk still starts from a
+// fresh state, so the cut does not show in the results.
+__device__ __forceinline__ bool find_run(const Problem &p, int C, uint32_t M, int rest, int slots, int &seq, int &c0, int &c1) {
+    int lo, hi;
+    if (p.nseq <= 64) {
+        const int lane_ = threadIdx.x & 63;
+        int first = 0, n = 0;
+        if (lane_ < p.nseq) {
+            const int p0 = tok_pos(p, lane_, 0), p1 = p0 + p.T - 1;
+            first = div_by(win_lo(p0, p.window), C, M);
+            n = p1 >= 0 ? max(0, min(div_by(p1, C, M), div_by(p.max_pos, C, M)) - first + 1) : 0;
+        }
+        const int total = __builtin_amdgcn_readlane(wave_scan64(n), 63);
+        if (total > slots && slots >= p.nseq) {
+            int k = n, incl = 0;                            // runs of this lane's sequence
+            for (int g = (total + slots - 1) / slots;; g++) {
+                k = (n + g - 1) / g;
+                incl = wave_scan64(k);
+                if (__builtin_amdgcn_readlane(incl, 63) <= slots) break;    // (at the latest with one run per sequence)
+            }
+            const unsigned long long hit = __ballot(incl > rest);
+            if (!hit) return false;
+            const int l = __builtin_ctzll(hit), r = rest - (incl - k);
+            const int a0 = first + (k > 0 ? r * n / k : 0), a1 = first + (k > 0 ? (r + 1) * n / k : 0);
+            seq = l;
+            c0 = __builtin_amdgcn_readlane(a0, l); c1 = __builtin_amdgcn_readlane(a1, l);
+            return true;
+        }
+    }
+    if (!find_item(p, C, M, rest, seq, c0, lo, hi)) return false;
+    c1 = c0 + 1;
+    return true;
+}
+
+// Upper bound of the (sequence, chunk) items of a launch: every chunk up to max_pos, or, under a sliding
+// window with consecutive token positions, the at most (window + T - 2) / chunk + 2 chunks a window of window + T - 1
+// keys meets (a 32K-key cache with a 1K window then launches 6 items per sequence and head, not 128).
+inline long long chunk_items_bound(const Problem &p, int chunk) {
+    long long per = p.max_pos / chunk + 1;
+    if (p.window > 0 && (p.T == 1 || p.pos_mode == 1)) {
+        const long long w = ((long long)p.window + p.T - 2) / chunk + 2;
+        if (w < per) per = w;
+    }
+    return per * p.nseq;
+}
+
+// Split-KV decode / verify / tree kernels. Verify and tree rows on 16-bit caches at HD <= 256: with slot_runs chunk by
+// chunk of each sequence (batch-invariant), otherwise in equal runs over the whole batch (depends on the batch).
 hipError_t launch_split(const Problem &p, int chunk, Partials &part, hipStream_t st, bool slot_runs = true);
 // Streaming decode kernel (T x GRP <= 16 rows per KV head, HD 128/256, 16-bit cache);
 // hipErrorNotSupported for other shapes. Writes chunk partials for launch_combine.
@@ -80,6 +218,10 @@ hipError_t launch_decode_f32(const Problem &p, int chunk, const Partials &part, 
 // Flash prefill kernel (waves split query rows, K/V tiles shared through LDS). kv_split = 0: one pass per row
 // tile writing O directly; kv_split > 0: keys cut at absolute multiples of kv_split, partials + combine.
 hipError_t launch_prefill(const Problem &p, int kv_split, const Partials &part, hipStream_t st);
+// Verify and tree runs on the prefill tile: up to `chunk` keys per work item, partials for launch_combine (16-bit caches,
+// HD 128 / 256, chunk a multiple of 64, consecutive tokens).
+bool verify_tile_supported(const Problem &p, int chunk);
+hipError_t launch_verify_tile(const Problem &p, int chunk, const Partials &part, hipStream_t st);
 // The key split chosen for kv_split = -1 (0: none).
 int prefill_auto_split(const Problem &p);
 size_t prefill_lds_bytes(int HD);   // dynamic LDS of the HD-wide prefill tile (W = 0)

@@ -30,8 +30,8 @@
 // the tile pairing or how the prompt is chunked (attention_flash_v2.cuh:13-18).
 //
 // Key splits (kv_split > 0) restrict each work item to the keys of one absolute split and write LSE partials for
-// launch_combine. Tree masks are not served here: the reference's ancestor mask covers at most 32 draft nodes
-// (attention_flash.cuh:177), and such short query runs go to the split kernel.
+// launch_combine. VER is the form for short query runs over long caches (verify, draft trees): the items are the key
+// chunks of a ragged batch, found on the device, and the mask takes the tree's ancestor bits (attention_flash.cuh:177).
 #include "attn_device.h"
 #include "attn_internal.h"
 #include <algorithm>
@@ -45,6 +45,7 @@ struct PrefArgs {
     Problem p;
     Partials part;
     int kv_split;      // 0: none
+    uint32_t split_m;  // div_magic(kv_split)
     int nht;           // half tiles (pair) or tiles per sequence
     int nsplit;        // key splits per sequence
     int tqh;           // tokens per half tile (pair) or per tile
@@ -56,6 +57,7 @@ struct PrefArgs {
     int fold;          // 1: fold each XCD's slots (two co-resident workgroups per CU take a long and a short item)
     int q_al;          // Q is 16-byte aligned
     int grp_mul;       // ceil(65536 / GRP): rho / GRP = rho * grp_mul >> 16 for rho < 128
+    int slots;         // verify: workgroups per (KV head, tile) that run at once
     int ways;          // XCDs that share one KV head's items (> 0), or minus the KV heads that share an XCD; 0: neither
 };
 
@@ -75,19 +77,25 @@ struct PrefCfg {
     static constexpr int SLOTS = HD / 8;                 // 16-byte slots per key row
     static constexpr int ROWB = HD * 2;                  // bytes per key row (16-bit operands)
     static constexpr int HALF = SK * ROWB;               // bytes of one K (or V) step tile
+    static constexpr int STAGE = 2 * HALF;               // K, then V, of one step
     static constexpr int NQL = RR * SLOTS / 64 / NW;     // 16-byte Q loads per thread
     static constexpr int NLR = SK * SLOTS / 64;          // 64-slot rows of a step tile (one per wave load)
     static constexpr int NLD = (NLR + NW - 1) / NW;      // 16-byte loads per thread per step (K and V each)
-    static constexpr size_t LDS_TILES = (size_t)4 * HALF;  // K stages 0 and 1, V stages 1 and 0
+    static constexpr size_t LDS_TILES = (size_t)2 * STAGE;
     static constexpr int XSTR = HD / KG + 4;             // merge exchange row stride (floats)
     // merge exchange: [row block][row group][owner key group][sender slot (KG-1)][16 rows][XSTR]
     static constexpr size_t LDS_MERGE = (size_t)RB * RG * KG * (KG - 1) * 16 * XSTR * 4;
     static constexpr size_t LDS_STATS = (size_t)2 * NW * RB * 16 * 4;
-    static constexpr size_t STATS_OFF = LDS_MERGE;       // merge statistics past the exchange (over the tiles)
-    static constexpr size_t LDS = LDS_TILES > LDS_MERGE + LDS_STATS ? LDS_TILES : LDS_MERGE + LDS_STATS;
+    // The merge statistics follow the exchange, over the tiles; verify runs put both past stage 0, which the next chunk's
+    // first step fills meanwhile.
+    static constexpr size_t merge_off(bool ver) { return ver ? STAGE : 0; }
+    static constexpr size_t lds(bool ver) {
+        return LDS_TILES > merge_off(ver) + LDS_MERGE + LDS_STATS ? LDS_TILES : merge_off(ver) + LDS_MERGE + LDS_STATS;
+    }
+    static constexpr size_t LDS = lds(false);
     static_assert((SK * SLOTS) % 64 == 0, "step loads");
-    static_assert((RR * SLOTS) % (64 * NW) == 0 && RR * ROWB <= 2 * HALF && HR % (64 / SLOTS) == 0, "Q tile in a stage");
-    static_assert(RG % 2 == 0 && (NSUB == 2 || (NSUB == 1 && RB == 1)), "row block layout");
+    static_assert((RR * SLOTS) % (64 * NW) == 0 && RR * ROWB <= STAGE && HR % (64 / SLOTS) == 0, "Q tile in a stage");
+    static_assert(NSUB == 2 || (NSUB == 1 && RB == 1), "row block layout");
     static_assert((KG == 2 || KG == 4) && DB % KG == 0, "key groups");
 };
 
@@ -123,9 +131,12 @@ __device__ __forceinline__ void lds_wait(T (&r)[N]) {
                      "+v"(r[6]), "+v"(r[7]) : [c] "n"(CNT) : "memory");
 }
 
-template <int HD, int RB, int RG, int KG_, int NSUB, int WPE, int KVT, int QT, int OT>
-__global__ void __launch_bounds__(RG * KG_ * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
-prefill_kernel(const PrefArgs a) {
+// One work item: the rows of tile (or pair) qi from the last of (sequence, KV head) over key split sp. Verify runs call it
+// for the splits [c0, c1) in turn: the first call loads the Q fragments qop, each call but the last requests the first step
+// of the next split before it merges.
+template <int HD, int RB, int RG, int KG_, int NSUB, int KVT, int QT, int OT, bool VER>
+__device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh, int qi, int sp, int c0, int c1,
+                                             u32x4 (&qop)[RB][HD / 32], unsigned char *smem) {
     using Cf = PrefCfg<HD, RB, RG, KG_, NSUB>;
     constexpr int KG = Cf::KG, SK = Cf::SK, KS = Cf::KS, DB = Cf::DB, NLD = Cf::NLD, DO = Cf::DO;
     constexpr int SLOTS = Cf::SLOTS, ROWB = Cf::ROWB, HR = Cf::HR;
@@ -133,27 +144,10 @@ prefill_kernel(const PrefArgs a) {
     constexpr bool DMA = KVT != DT_FP32;                 // 16-bit caches go straight to LDS
     using KE = typename Elem<KVT>::T;
     using QE = typename Elem<QT>::T;
-    extern __shared__ __align__(16) unsigned char smem[];
-    float *stm = reinterpret_cast<float *>(smem + Cf::STATS_OFF), *stl = stm + Cf::NW * RB * 16;
+    unsigned char *const xmem = smem + Cf::merge_off(VER);
+    float *stm = reinterpret_cast<float *>(xmem + Cf::LDS_MERGE), *stl = stm + Cf::NW * RB * 16;
 
     const Problem &p = a.p;
-    // XCD-aware work index: dispatch slot b runs on XCD b % 8, and the work items of one KV head (longest first) share
-    // an XCD, so that head's K/V stays in one L2. Fewer heads than XCDs: a head's items are dealt in turn to its
-    // `ways` XCDs; a multiple of 8 heads: an XCD takes its heads' items in turn; other counts: every head's longest
-    // items first, over all XCDs. Long items of every head start first in each case: with the longest half of a head on
-    // one XCD and the shortest on another, the 1377-token prompt of 24 q-heads over 4 KV heads took 75 instead of 56 us.
-    // With a.fold the local slot k is folded: slots k and k + per/2 - which the dispatcher places on the same CU when
-    // two workgroups fit a CU and the grid is one round - take the k-th longest and the k-th shortest item.
-    const int per = (int)gridDim.x / 8, k_loc = (int)blockIdx.x / 8, h_loc = (per + 1) / 2, xcd = (int)blockIdx.x % 8;
-    const int k_f = !a.fold || k_loc < h_loc ? k_loc : per - 1 - (k_loc - h_loc);
-    int head, item;                                                     // head = sequence * NKV + KV head
-    if (a.ways > 0) { head = xcd / a.ways; item = k_f * a.ways + xcd % a.ways; }
-    else if (a.ways < 0) { item = k_f / -a.ways; head = xcd + 8 * (k_f + item * a.ways); }
-    else { const int i = 8 * k_f + xcd; item = i / a.heads; head = i - item * a.heads; }
-    if (item >= a.nitems || head >= a.heads) return;
-    // (runtime divisions take ~200 cycles each: skipped where the launch makes them trivial)
-    const int seq = p.nseq > 1 ? head / p.NKV : 0, kvh = head - seq * p.NKV;
-    const int qi = a.nsplit > 1 ? item / a.nsplit : item, sp = item - qi * a.nsplit;
     const int GRP = a.grp;
 
     const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, ln = lane & 15;
@@ -163,7 +157,7 @@ prefill_kernel(const PrefArgs a) {
     const KE *Kb = kv_base<KE>(p, false, seq) + (size_t)kvh * HD;
     const KE *Vb = kv_base<KE>(p, true, seq) + (size_t)kvh * HD;
     // Prefill tokens are consecutive: token t of this sequence sits at position pbase + t.
-    const int pbase = __builtin_amdgcn_readfirstlane(p.pos_arr ? p.pos_arr[seq] : p.base);
+    const int pbase = __builtin_amdgcn_readfirstlane(VER ? tok_pos(p, seq, 0) : p.pos_arr ? p.pos_arr[seq] : p.base);
 
     // The work item's tokens: one tile, or two half tiles (longest first; an empty half has tok1 == tok0).
     const int ht0 = a.nht - 1 - qi, ht1 = a.pair && qi < ht0 ? qi : -1;
@@ -176,6 +170,8 @@ prefill_kernel(const PrefArgs a) {
     const int hi_b = pbase + tok1[0];                                   // one past the last key (clamp bound)
     int j_hi = hi_b;
     if (a.kv_split > 0) { j_lo = max(j_lo, sp * a.kv_split); j_hi = min(j_hi, (sp + 1) * a.kv_split); }
+    const bool fresh = !VER || sp == c0;
+    const bool none = VER && j_lo >= j_hi;                              // no row of the tile has keys in this chunk
     const int s0 = j_lo / SK, nsteps = j_lo < j_hi ? (j_hi - 1) / SK - s0 + 1 : 0;
 
     // Step loads: thread slot S = (wave*NLD + u)*64 + lane of a K (V) stage holds the 16-byte column
@@ -206,20 +202,22 @@ prefill_kernel(const PrefArgs a) {
     // Loads [u0, u1) of the thread's NLD slots (K and V each).
     // 16-bit caches: buffer loads straight into LDS over the byte range the workgroup may read (the ring, or the
     // keys below hi_b), so the rows past the last key of a step read as zeros (they are masked) without clamping.
+    // (Verify runs on a ring may end before it was ever filled: their lanes past the last key are sent out of range.)
     const uint32_t kv_bytes = p.kv_cap > 0 ? (uint32_t)p.kv_cap * krow_b
                                            : (uint32_t)(max(hi_b, 1) - 1) * krow_b + (uint32_t)(HD * sizeof(KE));
     const __amdgpu_buffer_rsrc_t krs = make_rsrc(Kb, kv_bytes), vrs = make_rsrc(Vb, kv_bytes);
     int it_cur = 0;                                                     // the step being computed
-    // Step k < 0 is a no-op step: every lane is out of range, so its loads write zeros into the stages of the step
-    // after (already consumed by every wave) and touch no memory; this keeps the issue points branch-free.
+    // Step k < 0 is a no-op step: every lane is out of range, so its loads write zeros into the stage of the step
+    // before (already consumed by every wave) and touch no memory; this keeps the issue points branch-free.
     // prep(k) forms a step's first byte offset and stages; issue_part(st, u0, u1) issues slots [u0, u1).
-    struct StepLd { unsigned char *kd, *vd; unsigned soff; int s; };
+    struct StepLd { unsigned char *kd, *vd; unsigned soff; int s, keys; };
     auto prep = [&](int k) {
         StepLd st;
         const int kst = k < 0 ? it_cur + 1 : k;
         st.s = s0 + kst;
-        st.kd = smem + (size_t)(kst % 2) * Cf::HALF;
-        st.vd = smem + (size_t)(3 - kst % 2) * Cf::HALF;
+        if constexpr (VER) st.keys = p.kv_cap > 0 ? hi_b - st.s * SK : SK;
+        st.kd = smem + (size_t)(kst % 2) * Cf::STAGE;
+        st.vd = st.kd + Cf::HALF;
         // (the range check covers the vector offset, which holds the step's offset too)
         st.soff = k < 0 ? kv_bytes : (unsigned)__builtin_amdgcn_readfirstlane((int)((unsigned)key_row(p, st.s * SK) * krow_b));
         return st;
@@ -242,25 +240,30 @@ prefill_kernel(const PrefArgs a) {
                 *reinterpret_cast<u32x4 *>(st.kd + (size_t)S * 16) = load8_op<KVT, F16>(reinterpret_cast<const KE *>(reinterpret_cast<const char *>(Kb) + koff));
                 *reinterpret_cast<u32x4 *>(st.vd + (size_t)S * 16) = load8_op<KVT, F16>(reinterpret_cast<const KE *>(reinterpret_cast<const char *>(Vb) + voff));
             } else {
-                buffer_load_lds16(krs, st.kd + (size_t)i * 1024, (int)koff);
-                buffer_load_lds16(vrs, st.vd + (size_t)i * 1024, (int)voff);
+                if (VER && st.keys < SK && (i * 64 + lane) / SLOTS >= st.keys) koff = voff = kv_bytes;
+                buffer_load_lds16<VER>(krs, st.kd + (size_t)i * 1024, (int)koff);
+                buffer_load_lds16<VER>(vrs, st.vd + (size_t)i * 1024, (int)voff);
             }
         }
     };
     auto issue = [&](int k) { issue_part(prep(k), 0, NLD); };
     // The next step's loads go out in four parts spread over the current step (between the QK batches, after
     // the softmax, between the PV batches): a workgroup's 8 waves issuing all of them at once stalled every wave
-    // on the vector memory pipe for about a thousand cycles per step.
+    // on the vector memory pipe for about a thousand cycles per step. (Verify runs wait for HBM, not for the pipe: all at
+    // once, at the start.)
     constexpr int NPART = 4, PPART = (NLD + NPART - 1) / NPART;
-    auto issue_pt = [&](const StepLd &st, int pt) { issue_part(st, pt * PPART, min(NLD, (pt + 1) * PPART)); };
-    if (nsteps > 0) issue(0);
+    auto issue_pt = [&](const StepLd &st, int pt) {
+        if (VER) { if (pt == 0) issue_part(st, 0, NLD); }
+        else issue_part(st, pt * PPART, min(NLD, (pt + 1) * PPART));
+    };
+    if (nsteps > 0 && fresh) issue(0);
 
     // The Q tile goes through LDS as well (16 bytes per lane of whole rows, where fragment loads straight from memory
     // touch 64 bytes of 16 rows each), in the stage that step 1 will fill, in the K layout: 16-byte column c of tile row R
     // in slot c ^ kswz(R), rows past the last as zeros. Row rho of a half tile is token rho / GRP, head rho % GRP.
-    unsigned char *qs = smem + Cf::HALF;
+    unsigned char *qs = smem + Cf::STAGE;
     auto tok_of = [&](int rho) { return (int)((unsigned)(rho * a.grp_mul) >> 16); };    // rho / GRP
-    {
+    if (fresh) {
         constexpr bool QDMA = QT != DT_FP32;
         f32x4 raw[QDMA ? 1 : Cf::NQL][2];
 #pragma unroll
@@ -298,10 +301,12 @@ prefill_kernel(const PrefArgs a) {
     const int hb = a.pair ? rg * RB * 16 / HR : 0;
     const int htok = tok0[hb], hrows = (tok1[hb] - tok0[hb]) * GRP;
     int lrow[RB], rpos[RB];
+    uint32_t anc[RB];                                                   // verify: tree masks of the rows (relative to pbase)
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
         lrow[rb] = rg * RB * 16 + rb * 16 - hb * HR;
         rpos[rb] = lrow[rb] + ln < hrows ? pbase + htok + tok_of(lrow[rb] + ln) : -1;
+        if constexpr (VER) anc[rb] = p.anc && rpos[rb] >= 0 ? p.anc[(size_t)seq * p.T + rpos[rb] - pbase] : 0u;
     }
     int wlo[RB], whi[RB], lo_max[RB], pos_min[RB];
     int wlo_all = INT_MAX, whi_all = -1;
@@ -312,7 +317,7 @@ prefill_kernel(const PrefArgs a) {
         if (lrow[rb] < rho1) {
             const int pf = pbase + htok + tok_of(lrow[rb]), pl = pbase + htok + tok_of(rho1 - 1);
             wlo[rb] = max(win_lo(pf, p.window), j_lo); whi[rb] = min(pl, j_hi - 1);
-            lo_max[rb] = win_lo(pl, p.window); pos_min[rb] = pf;
+            lo_max[rb] = win_lo(pl, p.window); pos_min[rb] = VER && p.anc ? pbase - 1 : pf;   // tree keys: per key
         }
         wlo_all = min(wlo_all, wlo[rb]); whi_all = max(whi_all, whi[rb]);
     }
@@ -329,14 +334,15 @@ prefill_kernel(const PrefArgs a) {
         }
     }
     // Q fragments: lane (row ln, group g) holds dims 32 ks + 8 g .. of its rows.
-    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    __syncthreads();
-    u32x4 qop[RB][KS];
+    if (fresh) {
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+        __syncthreads();
 #pragma unroll
-    for (int rb = 0; rb < RB; rb++)
+        for (int rb = 0; rb < RB; rb++)
 #pragma unroll
-        for (int ks = 0; ks < KS; ks++)
-            qop[rb][ks] = *reinterpret_cast<const u32x4 *>(qs + (rg * RB * 16 + rb * 16 + ln) * ROWB + (((4 * ks + g) ^ kswz(ln)) << 4));
+            for (int ks = 0; ks < KS; ks++)
+                qop[rb][ks] = *reinterpret_cast<const u32x4 *>(qs + (rg * RB * 16 + rb * 16 + ln) * ROWB + (((4 * ks + g) ^ kswz(ln)) << 4));
+    }
 
     // Per-lane LDS byte addresses inside a step stage (the key group's rows start at kg*KT). A slot index
     // occupies address bits 4.., and the row base has those bits clear, so "slot s ^ x" is an XOR on the
@@ -345,7 +351,7 @@ prefill_kernel(const PrefArgs a) {
     const unsigned lds0 = (unsigned)(uintptr_t)smem;
     const int vr = 4 * g + (ln >> 2);
     const unsigned kaddr = lds0 + (kg * Cf::KT + ln) * ROWB + ((g ^ kswz(ln)) << 4);
-    const unsigned vaddr = lds0 + 3 * Cf::HALF + (kg * Cf::KT + vr) * ROWB + 8 * (ln & 1) + ((((ln & 3) >> 1) ^ vswz(vr)) << 4);
+    const unsigned vaddr = lds0 + Cf::HALF + (kg * Cf::KT + vr) * ROWB + 8 * (ln & 1) + ((((ln & 3) >> 1) ^ vswz(vr)) << 4);
 
     // One step's work for this wave's row blocks: qk_softmax, then pv. QK: the K fragments of a sub-tile are read in batches (inline asm,
     // one wait per batch, so the reads are not serialised behind the MFMAs) and every row block runs its MFMA chain on
@@ -357,7 +363,7 @@ prefill_kernel(const PrefArgs a) {
         const int jw = (s0 + it) * SK + kg * Cf::KT;
         // Per-lane LDS bases, made opaque so that the XOR-swizzled fragment addresses are formed next to their
         // reads instead of being hoisted out of the step loop (which held ~30 address registers live and spilled).
-        unsigned kbase = kaddr + (it & 1) * Cf::HALF;
+        unsigned kbase = kaddr + (it & 1) * Cf::STAGE;
         asm volatile("" : "+v"(kbase));
         constexpr int NCH = NSUB == 1 ? 2 : 1;                          // independent MFMA chains per S fragment
         f32x4 s[NSUB][RB][NCH];
@@ -421,6 +427,16 @@ prefill_kernel(const PrefArgs a) {
 #pragma unroll
                     for (int i = 0; i < 4; i++)
                         if ((16 * sub + i < kl) | (16 * sub + i > kh)) tv[sub][rb][i] = kNegInf;
+                if (VER && p.anc) {
+                    const int d0 = jw + 4 * g - pbase;
+#pragma unroll
+                    for (int sub = 0; sub < NSUB; sub++)
+#pragma unroll
+                        for (int i = 0; i < 4; i++) {
+                            const int d = d0 + 16 * sub + i;
+                            if ((d >= 0) & ((d >= 32) | !((anc[rb] >> (d & 31)) & 1u))) tv[sub][rb][i] = kNegInf;
+                        }
+                }
             }
 #pragma unroll
             for (int sub = 0; sub < NSUB; sub++)
@@ -456,7 +472,7 @@ prefill_kernel(const PrefArgs a) {
     };
     auto pv = [&](int it, const StepLd &nxt) {
         int pt = NPART / 2;
-        unsigned vbase = vaddr - (it & 1) * Cf::HALF;
+        unsigned vbase = vaddr + (it & 1) * Cf::STAGE;
         asm volatile("" : "+v"(vbase));
         // PV with V^T fragments in batches of PB dim blocks, software-pipelined: batch b+1 is read before batch b's MFMAs.
         // As for K, the eight dim blocks that differ in the swizzled bits take an XOR of the base, the others (16-byte
@@ -539,6 +555,14 @@ prefill_kernel(const PrefArgs a) {
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) l[rb] = sum_over_groups(l[rb]);
     __syncthreads();                                                 // every wave is done with the K/V tiles
+    if (VER && sp + 1 < c1) {
+        StepLd nx;
+        nx.s = max(win_lo(pbase + tok0[0], p.window), (sp + 1) * a.kv_split) / SK; nx.kd = smem; nx.vd = smem + Cf::HALF;
+        nx.keys = p.kv_cap > 0 ? hi_b - nx.s * SK : SK;
+        nx.soff = (unsigned)__builtin_amdgcn_readfirstlane((int)((unsigned)key_row(p, nx.s * SK) * krow_b));
+        issue_part(nx, 0, NLD);
+    }
+    if (none) return;
 
     // Merge the KG key-group states of each row (waves kg = 0..KG-1 of a row group hold the same rows). Every
     // lane derives the row's M = max m and L = sum l 2^(m - M) (key groups in order) from the published (m, l)
@@ -551,7 +575,7 @@ prefill_kernel(const PrefArgs a) {
         for (int rb = 0; rb < RB; rb++) { stm[wave * RB * 16 + rb * 16 + ln] = m[rb]; stl[wave * RB * 16 + rb * 16 + ln] = l[rb]; }
     }
     __syncthreads();
-    float *xb = reinterpret_cast<float *>(smem);                        // exchange (reuses the tiles)
+    float *xb = reinterpret_cast<float *>(xmem);                        // exchange (reuses the tiles)
     auto xslot = [&](int rb, int owner, int sender) {
         return xb + ((((size_t)(rb * RG + rg) * KG + owner) * (KG - 1) + (sender < owner ? sender : sender - 1)) * 16 + ln) * Cf::XSTR + 4 * g;
     };
@@ -621,6 +645,44 @@ prefill_kernel(const PrefArgs a) {
     }
 }
 
+template <int HD, int RB, int RG, int KG_, int NSUB, int WPE, int KVT, int QT, int OT, bool VER>
+__global__ void __launch_bounds__(RG * KG_ * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
+prefill_kernel(const PrefArgs a) {
+    extern __shared__ __align__(16) unsigned char smem[];
+    const Problem &p = a.p;
+    int seq, kvh, qi;                                                   // sequence, KV head, tile from the last
+    if constexpr (VER) {
+        // Verify: runs of a sequence's key chunks, KV heads and tiles of one run side by side.
+        const int per = p.NKV * a.nht, it = (int)blockIdx.x / per, x = (int)blockIdx.x - it * per;
+        int c0, c1;
+        if (!find_run(p, a.kv_split, a.split_m, it, a.slots, seq, c0, c1)) return;
+        seq = __builtin_amdgcn_readfirstlane(seq); c0 = __builtin_amdgcn_readfirstlane(c0); c1 = __builtin_amdgcn_readfirstlane(c1);
+        qi = x / p.NKV; kvh = x - qi * p.NKV;
+        u32x4 qop[RB][HD / 32];
+        for (int sp = c0; sp < c1; sp++) prefill_item<HD, RB, RG, KG_, NSUB, KVT, QT, OT, true>(a, seq, kvh, qi, sp, c0, c1, qop, smem);
+    } else {
+        // XCD-aware work index: dispatch slot b runs on XCD b % 8, and the work items of one KV head (longest first) share
+        // an XCD, so that head's K/V stays in one L2. Fewer heads than XCDs: a head's items are dealt in turn to its
+        // `ways` XCDs; a multiple of 8 heads: an XCD takes its heads' items in turn; other counts: every head's longest
+        // items first, over all XCDs. Long items of every head start first in each case: with the longest half of a head on
+        // one XCD and the shortest on another, the 1377-token prompt of 24 q-heads over 4 KV heads took 75 instead of 56 us.
+        // With a.fold the local slot k is folded: slots k and k + per/2 - which the dispatcher places on the same CU when
+        // two workgroups fit a CU and the grid is one round - take the k-th longest and the k-th shortest item.
+        const int per = (int)gridDim.x / 8, k_loc = (int)blockIdx.x / 8, h_loc = (per + 1) / 2, xcd = (int)blockIdx.x % 8;
+        const int k_f = !a.fold || k_loc < h_loc ? k_loc : per - 1 - (k_loc - h_loc);
+        int head, item;                                                     // head = sequence * NKV + KV head
+        if (a.ways > 0) { head = xcd / a.ways; item = k_f * a.ways + xcd % a.ways; }
+        else if (a.ways < 0) { item = k_f / -a.ways; head = xcd + 8 * (k_f + item * a.ways); }
+        else { const int i = 8 * k_f + xcd; item = i / a.heads; head = i - item * a.heads; }
+        if (item >= a.nitems || head >= a.heads) return;
+        // (runtime divisions take ~200 cycles each: skipped where the launch makes them trivial)
+        seq = p.nseq > 1 ? head / p.NKV : 0; kvh = head - seq * p.NKV;
+        qi = a.nsplit > 1 ? item / a.nsplit : item;
+        u32x4 qop[RB][HD / 32];
+        prefill_item<HD, RB, RG, KG_, NSUB, KVT, QT, OT, false>(a, seq, kvh, qi, item - qi * a.nsplit, 0, 0, qop, smem);
+    }
+}
+
 // ---------------------------------------------------------------- host side
 // Tile shapes: 8 waves (two per SIMD) as 4 row groups x 2 key groups, 16 rows and HD accumulator columns per wave, a
 // 64-row workgroup tile, 64-key steps (two 16-key sub-tiles per wave) in two LDS stages. HD 512: 32-key steps (a 32-key
@@ -642,23 +704,28 @@ template <> struct PrefTile<256, 0> { static constexpr int RB = 1, RG = 4, KG = 
 template <> struct PrefTile<256, 1> { static constexpr int RB = 1, RG = 6, KG = 2, NSUB = 2, WPE = 3; };
 template <> struct PrefTile<256, 2> { static constexpr int RB = 2, RG = 4, KG = 2, NSUB = 2, WPE = 2; };
 template <> struct PrefTile<512, 0> { static constexpr int RB = 1, RG = 4, KG = 2, NSUB = 1, WPE = 2; };
+// W = 3, 4: verify runs, tiles of 32 and 64 rows.
+template <> struct PrefTile<128, 3> { static constexpr int RB = 1, RG = 2, KG = 2, NSUB = 2, WPE = 2; };
+template <> struct PrefTile<128, 4> { static constexpr int RB = 1, RG = 4, KG = 2, NSUB = 2, WPE = 4; };
+template <> struct PrefTile<256, 3> { static constexpr int RB = 1, RG = 2, KG = 2, NSUB = 2, WPE = 2; };
+template <> struct PrefTile<256, 4> { static constexpr int RB = 1, RG = 4, KG = 2, NSUB = 2, WPE = 2; };
 template <int HD, int W>
 using PrefTileCfg = PrefCfg<HD, PrefTile<HD, W>::RB, PrefTile<HD, W>::RG, PrefTile<HD, W>::KG,
                             PrefTile<HD, W>::NSUB>;
 
-template <int HD, int W, int KVT, int QT, int OT>
+template <int HD, int W, int KVT, int QT, int OT, bool VER = false>
 static hipError_t launch_pref_t(const PrefArgs &a, dim3 grid, hipStream_t st) {
     using T = PrefTile<HD, W>;
     using Cf = PrefTileCfg<HD, W>;
     static bool configured = false;
-    auto kern = prefill_kernel<HD, T::RB, T::RG, T::KG, T::NSUB, T::WPE, KVT, QT, OT>;
+    auto kern = prefill_kernel<HD, T::RB, T::RG, T::KG, T::NSUB, T::WPE, KVT, QT, OT, VER>;
     if (!configured) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
-                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)Cf::LDS);
+                                           hipFuncAttributeMaxDynamicSharedMemorySize, (int)Cf::lds(VER));
         if (e != hipSuccess) return e;
         configured = true;
     }
-    hipLaunchKernelGGL(kern, grid, dim3(Cf::NT), Cf::LDS, st, a);
+    hipLaunchKernelGGL(kern, grid, dim3(Cf::NT), Cf::lds(VER), st, a);
     return hipGetLastError();
 }
 
@@ -816,8 +883,8 @@ hipError_t launch_prefill(const Problem &p, int kv_split, const Partials &part, 
     const int fold = (per_cu >= 2 && nwg <= (long)per_cu * ncu) ? 1 : 0;
     const int ways = heads < 8 && 8 % heads == 0 ? 8 / heads : heads % 8 == 0 ? -(heads / 8) : 0;
     const long per = ways > 0 ? (nitems + ways - 1) / ways : (nwg + 7) / 8;
-    PrefArgs a{p, part, kv_split, pl.nht, nsplit, pl.tqh, pl.pair, (int)nitems, heads, GRP, p.scale * kLog2e, fold,
-               (reinterpret_cast<uintptr_t>(p.Q) & 15) == 0 ? 1 : 0, 65535 / GRP + 1, ways};
+    PrefArgs a{p, part, kv_split, 0u, pl.nht, nsplit, pl.tqh, pl.pair, (int)nitems, heads, GRP, p.scale * kLog2e, fold,
+               (reinterpret_cast<uintptr_t>(p.Q) & 15) == 0 ? 1 : 0, 65535 / GRP + 1, 0, ways};
     dim3 grid((unsigned)(8 * per));
     hipError_t e = hipErrorInvalidValue;
     const int kv = p.kv_dtype, q = p.q_dtype, o = p.o_dtype;
@@ -829,6 +896,45 @@ hipError_t launch_prefill(const Problem &p, int kv_split, const Partials &part, 
     else return hipErrorInvalidValue;
     if (e != hipSuccess || kv_split <= 0) return e;
     return launch_combine(p, kv_split, part, st);
+}
+
+// Verify and tree runs (more than 16 rows per KV head): the keys in absolute chunks, found on the device from the positions
+// (find_run), one partial per (row, chunk). Against a tile of four waves that each walk all 16-key tiles of the chunk, two
+// key groups and 64-key steps halve the chain of a chunk: a 7-token draft over 3001 keys (24 workgroups) takes 23.9 instead
+// of 47.1 us. 16 trees of 8 nodes over up to 16K keys (876 chunks, bound by HBM: 26 GB/s per CU inside the loop) take 131
+// against 133 us; one chunk per workgroup there 134. 32-key steps took 158 us with two stages (a step then is one HBM
+// latency) and 153 with four.
+bool verify_tile_supported(const Problem &p, int chunk) {
+    return (p.HD == 128 || p.HD == 256) && p.kv_dtype != DT_FP32 && (p.q_dtype == DT_FP32 || p.q_dtype == p.kv_dtype) &&
+           p.NQ % p.NKV == 0 && p.NQ / p.NKV <= 2 * pref_half_rows(p.HD) && chunk > 0 && chunk % 32 == 0 &&
+           (p.pos_mode == 1 || p.T == 1);
+}
+
+template <int KVT, int QT>
+static hipError_t verify_dispatch(const PrefArgs &a, bool narrow, dim3 grid, hipStream_t st) {
+    if (a.p.HD == 128)
+        return narrow ? launch_pref_t<128, 3, KVT, QT, DT_FP32, true>(a, grid, st)
+                      : launch_pref_t<128, 4, KVT, QT, DT_FP32, true>(a, grid, st);
+    return narrow ? launch_pref_t<256, 3, KVT, QT, DT_FP32, true>(a, grid, st)
+                  : launch_pref_t<256, 4, KVT, QT, DT_FP32, true>(a, grid, st);
+}
+
+hipError_t launch_verify_tile(const Problem &p, int chunk, const Partials &part, hipStream_t st) {
+    if (!verify_tile_supported(p, chunk)) return hipErrorNotSupported;
+    if (p.max_pos / chunk + 1 > part.ns_cap) return hipErrorInvalidValue;
+    const int GRP = p.NQ / p.NKV;
+    const bool narrow = (long)p.T * GRP <= 32;             // (a row's bits do not depend on the tile)
+    const int tq = (narrow ? 32 : 64) / GRP, nt = (p.T + tq - 1) / tq;
+    const long long wgs = chunk_items_bound(p, chunk) * p.NKV * nt;
+    if (wgs > INT_MAX) return hipErrorInvalidConfiguration;
+    PrefArgs a{p, part, chunk, div_magic(chunk), nt, 1, tq, 0, 0, p.nseq * p.NKV, GRP, p.scale * kLog2e, 0,
+               (reinterpret_cast<uintptr_t>(p.Q) & 15) == 0 ? 1 : 0, 65535 / GRP + 1,
+               std::max(1, device_cus() * (p.HD == 128 ? 2 : 1) / (p.NKV * nt)), 0};
+    const dim3 grid((unsigned)wgs);
+    const bool q32 = p.q_dtype == DT_FP32;
+    if (p.kv_dtype == DT_F16)
+        return q32 ? verify_dispatch<DT_F16, DT_FP32>(a, narrow, grid, st) : verify_dispatch<DT_F16, DT_F16>(a, narrow, grid, st);
+    return q32 ? verify_dispatch<DT_BF16, DT_FP32>(a, narrow, grid, st) : verify_dispatch<DT_BF16, DT_BF16>(a, narrow, grid, st);
 }
 
 }  // namespace dgx

@@ -1,11 +1,11 @@
-// Split-KV GQA attention for verify, speculative tree verify and the decode shapes the streaming decode kernel
-// does not take (fp32 caches, HD 512, more than 16 query heads per KV head) on gfx950.
+// Split-KV GQA attention for the decode shapes the streaming decode kernel does not take (fp32 caches, HD 512), the
+// equal-run mode of batched verify, and the LSE combine, on gfx950.
 //
 // Replaces the reference's attn_split_p1_kernel / attn_split_combine_kernel
 // (kernels/attention_decode_split.cuh:43-165) and, for short query runs, flash_attn2bs_p1(_custom)_kernel /
 // flash_attn2bs_p2_kernel (kernels/attention_flash.cuh:28-227).
 //
-// Grid: (kv head, chunk c, sequence x query-token tile). One workgroup = 4 wave64s. It owns the query rows
+// split_kernel. Grid: (kv head, chunk c, sequence x query-token tile). One workgroup = 4 wave64s. It owns the query rows
 // (token, head) of one KV head (GQA group, rows token-major, RB blocks of 16) for a token tile and the keys
 // [c*C, (c+1)*C) of its sequence, and writes one LSE partial per (row, chunk). The chunk's keys stream in
 // 16-key tiles at absolute positions:
@@ -18,15 +18,15 @@
 //     with the gfx950 transpose read (ds_read_b64_tr_b16), P^T straight from the softmax registers.
 // Every K/V byte of a chunk is read once per workgroup and serves all GRP query heads of the KV head.
 // With 2-4 row blocks (RB >= 2) wave w instead owns row block w with all head dims, so no S or PV work is repeated
-// across waves. For 16-bit caches at HD 128/256 those shapes (verify and tree verify runs) go to verify_kernel,
-// the same layout fed by a four-stage direct-to-LDS ring (global_load_lds, no staging registers) over a grid of
-// resident workgroups that each stream an equal run of key tiles (see seg_scan).
+// across waves. For 16-bit caches at HD 128/256 those shapes (verify and tree verify runs) go to the verify form of the
+// prefill tile, or in the equal-run mode to verify_kernel: the same layout fed by a four-stage direct-to-LDS ring
+// (global_load_lds, no staging registers) over a grid of resident workgroups that each stream an equal run of key tiles
+// (see seg_scan).
 //
 // Invariants (kept from the reference, attention_decode_split.cuh:8-12) for split_kernel: chunk and tile
 // boundaries are absolute key positions and the chunk combine runs in fixed order. A row's result therefore does
 // not depend on the batch, the other rows of its tile, the grid size or the maximum position: a row is
-// bit-identical alone or as a batch row. verify_kernel keeps this in its default mode (slot_runs: partials at
-// absolute key chunks of each sequence); its other mode gives it up for equal runs (boundaries that follow the total
+// bit-identical alone or as a batch row. verify_kernel's equal runs give this up (boundaries that follow the total
 // key count), deterministic for given inputs.
 #include "attn_device.h"
 #include "attn_internal.h"
@@ -43,7 +43,6 @@ struct SplitArgs {
     int tpb;        // query tokens per workgroup
     int nchunks;    // token tiles per sequence
     float sl2;      // scale * log2(e)
-    int slot_runs = 1;   // verify_kernel: 1 = runs are each pair's absolute key chunks (batch-invariant), 0 = equal runs
 };
 
 // Wave-wide reductions over all 64 lanes (fixed xor-butterfly order, identical result in every lane).
@@ -64,11 +63,6 @@ __device__ __forceinline__ float wave_sum(float v) {
 // writes one partial per pair it meets, into slot (run index - index of the pair's first run); the last run of a
 // pair marks the slot after its own for the combine. q depends on the total tile count, so verify results depend
 // on the batch; they are deterministic for given inputs.
-// With slot_runs (the default) each cut moves forward to the next absolute key-chunk boundary of its pair (C keys),
-// and a run flushes its state into partial slot (key / C) at every chunk boundary it crosses: the float operations
-// of a chunk then start from a fresh state at the chunk's first key whatever run holds it, so a row's result
-// depends only on its own sequence (the combine reads slots lo / C .. pos / C as for split_kernel). The cost is the
-// cut granularity: runs differ by up to C keys.
 struct SegPair { int seq, tok0, tok1, lo, hi, jb, n; };
 
 __device__ __forceinline__ SegPair seg_pair(const Problem &p, int tpb, int nchunks, int z) {
@@ -750,17 +744,9 @@ __device__ __forceinline__ void verify_segment(const SplitArgs &a, const SegPair
 #pragma unroll
             for (int j = 0; j < 8; j++) acc[d8 + j] = mfma_pv16<F16>(v[j], pop, acc[d8 + j]);
         }
-        if (a.slot_runs && it + 1 < ntile && (jt + KT) % a.C == 0) {
-            // The tile ends an absolute key chunk: its partial goes to slot (chunk index), the next chunk starts
-            // from a fresh state (the same float operations as a run that starts at that chunk).
-            write(jt / a.C, false);
-            m = kNegInf; l = 0.f;
-#pragma unroll
-            for (int db = 0; db < DB; db++) acc[db] = f32x4{0.f, 0.f, 0.f, 0.f};
-        }
     }
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");        // no load may land after the workgroup ends
-    write(a.slot_runs ? (jb + KT * (ntile - 1)) / a.C : slot, last && !a.slot_runs);
+    write(slot, last);
 }
 
 template <int HD, int RB, int KVT, int QT>
@@ -805,37 +791,15 @@ __global__ void __launch_bounds__(256) verify_kernel(const SplitArgs a) {
             seg_scan(p, a.tpb, a.nchunks, x, 0, n_, z, P, pz);
         }
     };
-    int x, x1;
-    if (a.slot_runs) {
-        // Equal runs, each end moved forward to the next absolute key-chunk boundary of its pair (or the pair's
-        // end): every chunk of a pair falls in one run, which writes it to partial slot (first key / C).
-        const int q = (N + G1 - 1) / G1, C = a.C;
-        auto snap = [&](long long xl) -> int {
-            if (xl >= N) return N;
-            const int xx = (int)xl;
-            locate(xx);
-            const int t = xx - P;
-            if (t == 0) return xx;
-            const SegPair s = pair_at(z);
-            const int kb = (s.jb + 16 * t + C - 1) / C * C;
-            return P + min((kb - s.jb) / 16, s.n);
-        };
-        x1 = snap((long long)(run + 1) * q);
-        x = snap((long long)run * q);
-        if (x >= x1) return;
-        locate(x);                                        // the snap may have moved x to the next pair
-    } else {
-        const int q = max((N + G1 - 1) / G1, a.part.seg_qmin);
-        const long long xs = (long long)run * q;
-        if (xs >= N) return;
-        x = (int)xs;
-        x1 = (int)min((long long)N, xs + q);
-        locate(x);
-    }
     const int q = max((N + G1 - 1) / G1, a.part.seg_qmin);
+    const long long xs = (long long)run * q;
+    if (xs >= N) return;
+    int x = (int)xs;
+    const int x1 = (int)min((long long)N, xs + q);
+    locate(x);
     SegPair sp = pair_at(z);
     for (;;) {
-        const int t0 = x - P, t1 = min(sp.n, t0 + (x1 - x)), slot = a.slot_runs ? 0 : run - P / q;
+        const int t0 = x - P, t1 = min(sp.n, t0 + (x1 - x)), slot = run - P / q;
         if (slot < 0 || slot >= a.part.ns_cap) break;     // unreachable while the counts agree
         if (t0 >= t1) break;                              // unreachable: x lies inside pair z
         verify_segment<HD, RB, KVT, QT>(a, sp, kvh, t0, t1, slot, t1 == sp.n, smem);
@@ -880,9 +844,9 @@ static hipError_t verify_grid(int &G) {
 }
 
 template <int HD, int RB, int KVT, int QT>
-static hipError_t launch_split_t(SplitArgs &a, dim3 grid, hipStream_t st) {
+static hipError_t launch_split_t(SplitArgs &a, dim3 grid, bool equal_runs, hipStream_t st) {
     if constexpr (RB >= 2 && HD <= 256 && KVT != DT_FP32) {
-        if (a.part.ns_cap >= 2) {
+        if (equal_runs && a.part.ns_cap >= 2) {
             int G = 0;
             hipError_t e = verify_grid<HD, RB, KVT, QT>(G);
             if (e != hipSuccess) return e;
@@ -890,10 +854,8 @@ static hipError_t launch_split_t(SplitArgs &a, dim3 grid, hipStream_t st) {
             // floor((n - 1) / q) + 2 runs (with fewer than ns_cap, the slot after the last holds the end mark).
             const int nmax = a.p.max_pos / 16 + 1;
             G = std::max(a.p.NKV, G - G % a.p.NKV);          // the same G / NKV runs for every KV head
-            if (!a.slot_runs) {
-                a.part.seg_g = G;
-                a.part.seg_qmin = std::max(8, (nmax - 1) / (a.part.ns_cap - 1) + 1);
-            }
+            a.part.seg_g = G;
+            a.part.seg_qmin = std::max(8, (nmax - 1) / (a.part.ns_cap - 1) + 1);
             hipLaunchKernelGGL((verify_kernel<HD, RB, KVT, QT>), dim3(G), dim3(256), VerifyCfg<HD>::LDS, st, a);
             return hipGetLastError();
         }
@@ -911,22 +873,22 @@ static hipError_t launch_split_t(SplitArgs &a, dim3 grid, hipStream_t st) {
 }
 
 template <int HD, int KVT, int QT>
-static hipError_t dispatch_rb(SplitArgs &a, int RB, dim3 grid, hipStream_t st) {
+static hipError_t dispatch_rb(SplitArgs &a, int RB, dim3 grid, bool eq, hipStream_t st) {
     switch (RB) {
-    case 1: return launch_split_t<HD, 1, KVT, QT>(a, grid, st);
-    case 2: return launch_split_t<HD, 2, KVT, QT>(a, grid, st);
-    case 3: return launch_split_t<HD, 3, KVT, QT>(a, grid, st);
-    case 4: return launch_split_t<HD, 4, KVT, QT>(a, grid, st);
+    case 1: return launch_split_t<HD, 1, KVT, QT>(a, grid, eq, st);
+    case 2: return launch_split_t<HD, 2, KVT, QT>(a, grid, eq, st);
+    case 3: return launch_split_t<HD, 3, KVT, QT>(a, grid, eq, st);
+    case 4: return launch_split_t<HD, 4, KVT, QT>(a, grid, eq, st);
     default: return hipErrorInvalidValue;
     }
 }
 
 template <int KVT, int QT>
-static hipError_t dispatch_hd(SplitArgs &a, int RB, dim3 grid, hipStream_t st) {
+static hipError_t dispatch_hd(SplitArgs &a, int RB, dim3 grid, bool eq, hipStream_t st) {
     switch (a.p.HD) {
-    case 128: return dispatch_rb<128, KVT, QT>(a, RB, grid, st);
-    case 512: return dispatch_rb<512, KVT, QT>(a, RB, grid, st);
-    case 256: return dispatch_rb<256, KVT, QT>(a, RB, grid, st);
+    case 128: return dispatch_rb<128, KVT, QT>(a, RB, grid, eq, st);
+    case 512: return dispatch_rb<512, KVT, QT>(a, RB, grid, eq, st);
+    case 256: return dispatch_rb<256, KVT, QT>(a, RB, grid, eq, st);
     default: return hipErrorInvalidValue;
     }
 }
@@ -953,23 +915,24 @@ hipError_t launch_split(const Problem &p, int chunk, Partials &part, hipStream_t
     // Up to 16 rows per KV head (one query token at GRP <= 16): the streaming decode kernel.
     if (decode_stream_supported(p))
         return launch_decode_stream(p, chunk, part, st);
+    if (slot_runs && verify_tile_supported(p, chunk)) return launch_verify_tile(p, chunk, part, st);
     if (p.NQ % p.NKV) return hipErrorInvalidValue;
     const int GRP = p.NQ / p.NKV;
     int RB, tpb, nchunks;
     split_tiling(p, RB, tpb, nchunks);
     if (RB * 16 < GRP || RB > 4) return hipErrorInvalidValue;
     if (p.max_pos / chunk + 1 > part.ns_cap) return hipErrorInvalidValue;
-    SplitArgs a{p, part, chunk, tpb, nchunks, p.scale * kLog2e, slot_runs ? 1 : 0};
+    SplitArgs a{p, part, chunk, tpb, nchunks, p.scale * kLog2e};
     dim3 grid(p.NKV, p.max_pos / chunk + 1, p.nseq * nchunks);
     if (grid.z > 65535u || grid.y > 65535u) return hipErrorInvalidConfiguration;
     if ((long long)p.nseq * p.NKV * (p.max_pos / 16 + 2) > INT_MAX) return hipErrorInvalidConfiguration;
     const int kv = p.kv_dtype, q = p.q_dtype;
     hipError_t e = hipErrorInvalidValue;
-    if (kv == DT_F16 && q == DT_FP32) e = dispatch_hd<DT_F16, DT_FP32>(a, RB, grid, st);
-    else if (kv == DT_F16 && q == DT_F16) e = dispatch_hd<DT_F16, DT_F16>(a, RB, grid, st);
-    else if (kv == DT_BF16 && q == DT_FP32) e = dispatch_hd<DT_BF16, DT_FP32>(a, RB, grid, st);
-    else if (kv == DT_BF16 && q == DT_BF16) e = dispatch_hd<DT_BF16, DT_BF16>(a, RB, grid, st);
-    else if (kv == DT_FP32 && q == DT_FP32) e = dispatch_hd<DT_FP32, DT_FP32>(a, RB, grid, st);
+    if (kv == DT_F16 && q == DT_FP32) e = dispatch_hd<DT_F16, DT_FP32>(a, RB, grid, !slot_runs, st);
+    else if (kv == DT_F16 && q == DT_F16) e = dispatch_hd<DT_F16, DT_F16>(a, RB, grid, !slot_runs, st);
+    else if (kv == DT_BF16 && q == DT_FP32) e = dispatch_hd<DT_BF16, DT_FP32>(a, RB, grid, !slot_runs, st);
+    else if (kv == DT_BF16 && q == DT_BF16) e = dispatch_hd<DT_BF16, DT_BF16>(a, RB, grid, !slot_runs, st);
+    else if (kv == DT_FP32 && q == DT_FP32) e = dispatch_hd<DT_FP32, DT_FP32>(a, RB, grid, !slot_runs, st);
     part = a.part;                                     // the combine reads how the partials were laid out
     return e;
 }
