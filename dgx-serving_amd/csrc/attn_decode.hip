@@ -279,8 +279,12 @@ static hipError_t launch_dec_e(const DecodeArgs &a, dim3 grid, hipStream_t st) {
 }
 template <int HD, int RW, int KVT, int QT>
 static hipError_t launch_dec_rw(const DecodeArgs &a, dim3 grid, hipStream_t st) {
-    // (the choice depends on the layer only, so a row's bits do not depend on the batch)
-    if (a.p.window > 0) return launch_dec_e<HD, RW, KVT, QT, true>(a, grid, st);
+    // Early refill (the same float operations in the same order) for sliding windows, and at HD 256 for launches of at most
+    // two workgroups per CU of a 256-CU device: there no other wave covers a tile's load. A one-token step of 3 sequences
+    // over up to 2.9K keys takes 20.8 instead of 23.8 us, 6 over up to 538 29.9 instead of 32.5; the 564-workgroup batch
+    // of 16 stays at 57.8 either way, and at HD 128 it gains nothing (13.8 against 13.5 us for one sequence of 512 keys).
+    // Two tiles ahead (254 VGPRs, one wave per SIMD) took 22.5 and 31.1 us.
+    if (a.p.window > 0 || (HD == 256 && grid.x <= 512u)) return launch_dec_e<HD, RW, KVT, QT, true>(a, grid, st);
     return launch_dec_e<HD, RW, KVT, QT, false>(a, grid, st);
 }
 

@@ -95,8 +95,9 @@ __device__ __forceinline__ int wave_scan64(int v) {
 // index order and a CU that receives more workgroups than the others shares its bandwidth among them, so the short
 // items go last, where they land on the CUs that get a third workgroup (measured: a CU with three full items runs
 // 20% longer than one with two).
-// Up to 64 sequences take one position load, one scan and no division; the general form is ~2 us (its scans go through
-// LDS shuffles), which a workgroup spends before its first load.
+// The divisions by C are multiplications and the scans run on the VALU (2.2 -> about 1 us before a workgroup's first load).
+// A form without the second pass over the positions starts the short items of phase 1 as early as the others, and the
+// 564-workgroup decode batch is then slower (57.9 against 57.5 us).
 __device__ __forceinline__ bool find_item(const Problem &p, int C, uint32_t M, int rest, int &seq, int &c, int &lo, int &hi) {
     const int lane_ = threadIdx.x & 63, cmax = div_by(p.max_pos, C, M);
     seq = -1; c = 0;
@@ -117,26 +118,6 @@ __device__ __forceinline__ bool find_item(const Problem &p, int C, uint32_t M, i
         const int kf = min(hi_s, (first + 1) * C) - lo_s, kl = hi_s - max(lo_s, (first + n - 1) * C);
         return n >= 2 && kf >= kl ? n - 1 : 0;
     };
-    if (p.nseq <= 64) {
-        int lo_s = 0, hi_s = 0, first = 0, n = 0;
-        if (lane_ < p.nseq) range(lane_, lo_s, hi_s, first, n);
-        const int m = max(n - 1, 0), incl = wave_scan64(m), total = __builtin_amdgcn_readlane(incl, 63);
-        unsigned long long hit;
-        if (rest < total) {
-            hit = __ballot(incl > rest);
-        } else {                                            // the (rest - total)-th sequence with keys
-            const unsigned long long some = __ballot(n > 0);
-            const int rank = __builtin_amdgcn_mbcnt_hi((unsigned)(some >> 32), __builtin_amdgcn_mbcnt_lo((unsigned)some, 0));
-            hit = __ballot(n > 0 && rank == rest - total);
-            if (!hit) return false;
-        }
-        const int l = __builtin_ctzll(hit);
-        const int sh = short_chunk(lo_s, hi_s, first, n), r = rest - (incl - m);    // of lane l: its own
-        const int cc = first + (rest >= total ? sh : r < sh ? r : r + 1);
-        seq = l;
-        c = __builtin_amdgcn_readlane(cc, l); lo = __builtin_amdgcn_readlane(lo_s, l); hi = __builtin_amdgcn_readlane(hi_s, l);
-        return true;
-    }
     for (int phase = 0; phase < 2; phase++) {
         for (int s0 = 0; s0 < p.nseq; s0 += 64) {
             int lo_s = 0, hi_s = 0, first = 0, n = 0;
