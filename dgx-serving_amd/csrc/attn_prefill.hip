@@ -564,36 +564,48 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
     }
     if (none) return;
 
-    // Merge the KG key-group states of each row (waves kg = 0..KG-1 of a row group hold the same rows). Every
-    // lane derives the row's M = max m and L = sum l 2^(m - M) (key groups in order) from the published (m, l)
-    // and scales its accumulator by 2^(m - M) / L (2^(m - M) for a split partial). Key group kg then owns output
-    // dim blocks [kg*DO, (kg+1)*DO): it parks the other groups' blocks of its scaled accumulator in LDS, and sums
-    // its own blocks over the key groups in order 0..KG-1 (the same order for every row and tiling).
+    // Merge the KG key-group states of each row (waves kg = 0..KG-1 of a row group hold the same rows). Key group kg owns
+    // output dim blocks [kg*DO, (kg+1)*DO): every wave publishes its rows' (m, l) and parks the other groups' blocks of its
+    // accumulator in LDS; after one barrier every lane derives M = max m and L = sum l 2^(m - M) (key groups in order) and
+    // sums its own blocks over the key groups in order 0..KG-1 (the same order for every row and tiling), each scaled by
+    // 2^(m - M) / L (2^(m - M) for a split partial).
     const int NQ = p.NQ;
     if (g == 0) {
 #pragma unroll
         for (int rb = 0; rb < RB; rb++) { stm[wave * RB * 16 + rb * 16 + ln] = m[rb]; stl[wave * RB * 16 + rb * 16 + ln] = l[rb]; }
     }
-    __syncthreads();
     float *xb = reinterpret_cast<float *>(xmem);                        // exchange (reuses the tiles)
     auto xslot = [&](int rb, int owner, int sender) {
         return xb + ((((size_t)(rb * RG + rg) * KG + owner) * (KG - 1) + (sender < owner ? sender : sender - 1)) * 16 + ln) * Cf::XSTR + 4 * g;
     };
-    float f[RB];
+    // park the blocks of the other owners (constant indices keep acc in registers)
+#pragma unroll
+    for (int rb = 0; rb < RB; rb++)
+        static_for<KG>([&](auto o_c) {
+            constexpr int O = decltype(o_c)::value;
+            if (O == kg) return;
+            float *dst = xslot(rb, O, kg);
+#pragma unroll
+            for (int j = 0; j < DO; j++) *reinterpret_cast<f32x4 *>(dst + 16 * j) = acc[rb][O * DO + j];
+        });
+    __syncthreads();
+    float f[RB][KG];                                                    // the key groups' factors
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
-        const int srow = rb * 16 + ln;
-        float M = kNegInf;
+        float M = kNegInf, mk[KG];
 #pragma unroll
-        for (int k = 0; k < KG; k++) M = fmaxf(M, stm[(rg * KG + k) * RB * 16 + srow]);
+        for (int k = 0; k < KG; k++) { mk[k] = stm[(rg * KG + k) * RB * 16 + rb * 16 + ln]; M = fmaxf(M, mk[k]); }
         float L = 0.f;
 #pragma unroll
         for (int k = 0; k < KG; k++) {
-            const float mk = stm[(rg * KG + k) * RB * 16 + srow];
-            if (mk != kNegInf) L += stl[(rg * KG + k) * RB * 16 + srow] * fast_exp2(mk - M);
+            f[rb][k] = mk[k] == kNegInf ? 0.f : fast_exp2(mk[k] - M);
+            if (mk[k] != kNegInf) L += stl[(rg * KG + k) * RB * 16 + rb * 16 + ln] * f[rb][k];
         }
-        f[rb] = (m[rb] == kNegInf) ? 0.f : fast_exp2(m[rb] - M);
-        if (a.kv_split <= 0) f[rb] *= (L > 0.f ? 1.f / L : 0.f);
+        if (a.kv_split <= 0) {
+            const float inv = L > 0.f ? 1.f / L : 0.f;
+#pragma unroll
+            for (int k = 0; k < KG; k++) f[rb][k] *= inv;
+        }
         const int rho = lrow[rb] + ln;
         if (kg == 0 && g == 0 && rho < hrows) {
             const int t = tok_of(rho), r = seq * p.T + htok + t, h = kvh * GRP + rho - t * GRP;
@@ -604,16 +616,7 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
                 p.lse[(size_t)r * NQ + h] = (L > 0.f) ? (M + log2f(L)) * kLn2 : kNegInf;
             }
         }
-        // park the blocks of the other owners (constant indices keep acc in registers)
-        static_for<KG>([&](auto o_c) {
-            constexpr int O = decltype(o_c)::value;
-            if (O == kg) return;
-            float *dst = xslot(rb, O, kg);
-#pragma unroll
-            for (int j = 0; j < DO; j++) *reinterpret_cast<f32x4 *>(dst + 16 * j) = acc[rb][O * DO + j] * f[rb];
-        });
     }
-    __syncthreads();
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
         const int rho = lrow[rb] + ln;
@@ -628,7 +631,7 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
                 f32x4 o = f32x4{0.f, 0.f, 0.f, 0.f};
 #pragma unroll
                 for (int k = 0; k < KG; k++) {
-                    const f32x4 x = k == O ? acc[rb][O * DO + j] * f[rb] : *reinterpret_cast<const f32x4 *>(xslot(rb, O, k) + 16 * j);
+                    const f32x4 x = (k == O ? acc[rb][O * DO + j] : *reinterpret_cast<const f32x4 *>(xslot(rb, O, k) + 16 * j)) * f[rb][k];
                     o = k == 0 ? x : o + x;
                 }
                 const int d = 16 * (O * DO + j) + 4 * g;
@@ -704,11 +707,10 @@ template <> struct PrefTile<256, 0> { static constexpr int RB = 1, RG = 4, KG = 
 template <> struct PrefTile<256, 1> { static constexpr int RB = 1, RG = 6, KG = 2, NSUB = 2, WPE = 3; };
 template <> struct PrefTile<256, 2> { static constexpr int RB = 2, RG = 4, KG = 2, NSUB = 2, WPE = 2; };
 template <> struct PrefTile<512, 0> { static constexpr int RB = 1, RG = 4, KG = 2, NSUB = 1, WPE = 2; };
-// W = 3, 4: verify runs, tiles of 32 and 64 rows.
-template <> struct PrefTile<128, 3> { static constexpr int RB = 1, RG = 2, KG = 2, NSUB = 2, WPE = 2; };
-template <> struct PrefTile<128, 4> { static constexpr int RB = 1, RG = 4, KG = 2, NSUB = 2, WPE = 4; };
-template <> struct PrefTile<256, 3> { static constexpr int RB = 1, RG = 2, KG = 2, NSUB = 2, WPE = 2; };
-template <> struct PrefTile<256, 4> { static constexpr int RB = 1, RG = 4, KG = 2, NSUB = 2, WPE = 2; };
+// W = 3: verify runs (also for 17-32 rows: a 32-row tile of four waves took 128 against 118 us for 12 sequences x 12 tokens
+// of 16 q-heads over 8, for its slower K/V requests).
+template <> struct PrefTile<128, 3> { static constexpr int RB = 1, RG = 4, KG = 2, NSUB = 2, WPE = 4; };
+template <> struct PrefTile<256, 3> { static constexpr int RB = 1, RG = 4, KG = 2, NSUB = 2, WPE = 2; };
 template <int HD, int W>
 using PrefTileCfg = PrefCfg<HD, PrefTile<HD, W>::RB, PrefTile<HD, W>::RG, PrefTile<HD, W>::KG,
                             PrefTile<HD, W>::NSUB>;
@@ -911,20 +913,16 @@ bool verify_tile_supported(const Problem &p, int chunk) {
 }
 
 template <int KVT, int QT>
-static hipError_t verify_dispatch(const PrefArgs &a, bool narrow, dim3 grid, hipStream_t st) {
-    if (a.p.HD == 128)
-        return narrow ? launch_pref_t<128, 3, KVT, QT, DT_FP32, true>(a, grid, st)
-                      : launch_pref_t<128, 4, KVT, QT, DT_FP32, true>(a, grid, st);
-    return narrow ? launch_pref_t<256, 3, KVT, QT, DT_FP32, true>(a, grid, st)
-                  : launch_pref_t<256, 4, KVT, QT, DT_FP32, true>(a, grid, st);
+static hipError_t verify_dispatch(const PrefArgs &a, dim3 grid, hipStream_t st) {
+    return a.p.HD == 128 ? launch_pref_t<128, 3, KVT, QT, DT_FP32, true>(a, grid, st)
+                         : launch_pref_t<256, 3, KVT, QT, DT_FP32, true>(a, grid, st);
 }
 
 hipError_t launch_verify_tile(const Problem &p, int chunk, const Partials &part, hipStream_t st) {
     if (!verify_tile_supported(p, chunk)) return hipErrorNotSupported;
     if (p.max_pos / chunk + 1 > part.ns_cap) return hipErrorInvalidValue;
     const int GRP = p.NQ / p.NKV;
-    const bool narrow = (long)p.T * GRP <= 32;             // (a row's bits do not depend on the tile)
-    const int tq = (narrow ? 32 : 64) / GRP, nt = (p.T + tq - 1) / tq;
+    const int tq = 64 / GRP, nt = (p.T + tq - 1) / tq;
     const long long wgs = chunk_items_bound(p, chunk) * p.NKV * nt;
     if (wgs > INT_MAX) return hipErrorInvalidConfiguration;
     PrefArgs a{p, part, chunk, div_magic(chunk), nt, 1, tq, 0, 0, p.nseq * p.NKV, GRP, p.scale * kLog2e, 0,
@@ -933,8 +931,8 @@ hipError_t launch_verify_tile(const Problem &p, int chunk, const Partials &part,
     const dim3 grid((unsigned)wgs);
     const bool q32 = p.q_dtype == DT_FP32;
     if (p.kv_dtype == DT_F16)
-        return q32 ? verify_dispatch<DT_F16, DT_FP32>(a, narrow, grid, st) : verify_dispatch<DT_F16, DT_F16>(a, narrow, grid, st);
-    return q32 ? verify_dispatch<DT_BF16, DT_FP32>(a, narrow, grid, st) : verify_dispatch<DT_BF16, DT_BF16>(a, narrow, grid, st);
+        return q32 ? verify_dispatch<DT_F16, DT_FP32>(a, grid, st) : verify_dispatch<DT_F16, DT_F16>(a, grid, st);
+    return q32 ? verify_dispatch<DT_BF16, DT_FP32>(a, grid, st) : verify_dispatch<DT_BF16, DT_BF16>(a, grid, st);
 }
 
 }  // namespace dgx

@@ -32,14 +32,16 @@ def _ref(Q, K, V, base, window, anc):
 
 
 # T x GRP rows: 17 (one past a block), 32, 33 (past the narrow tile), 48, 64, 65 and 96 (two token tiles), 200, 36 (GRP 36)
+SHAPES = [(17, 1, 1, 256), (16, 2, 1, 128), (11, 6, 2, 256), (8, 24, 4, 256), (16, 16, 4, 128), (13, 10, 2, 256),
+          (16, 24, 4, 256), (25, 16, 2, 128), (1, 36, 1, 256)]
+# 24 sequences of 64-key chunks are more items than run at once: a workgroup takes several chunks in turn; 70 sequences
+# (the smaller shapes) are more than a wave's lanes.
+BATCHES = [(1, 64, 0), (3, 96, 0), (70, 256, 0), (5, 160, 100), (24, 64, 0), (24, 64, 300)]
+
+
 @pytest.mark.parametrize("kvdt", [1, 2])
-@pytest.mark.parametrize("T,nq,nkv,hd", [(17, 1, 1, 256), (16, 2, 1, 128), (11, 6, 2, 256), (8, 24, 4, 256), (16, 16, 4, 128),
-                                         (13, 10, 2, 256), (16, 24, 4, 256), (25, 16, 2, 128), (1, 36, 1, 256)])
-# 24 sequences of 64-key chunks are more items than run at once: a workgroup takes several chunks in turn
-@pytest.mark.parametrize("B,chunk,window", [(1, 64, 0), (3, 96, 0), (70, 256, 0), (5, 160, 100), (24, 64, 0), (24, 64, 300)])
+@pytest.mark.parametrize("T,nq,nkv,hd,B,chunk,window", [s + b for s in SHAPES for b in BATCHES if b[0] < 70 or s[0] * s[1] <= 200])
 def test_verify_tile_against_fp32(T, nq, nkv, hd, kvdt, B, chunk, window):
-    if B == 70 and T * nq > 200:
-        pytest.skip("the many-sequence enumeration is covered by the smaller shapes")
     rng = np.random.default_rng(T * 100 + B)
     base = rng.integers(0, 700, B).astype(np.int32)
     base[0] = (0, 63, 64, 95, 160)[B % 5]                   # around step and chunk edges
