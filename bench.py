@@ -130,7 +130,7 @@ def run_tree(steps, warmup, seed=5, runs=None):
     max_pos = int(committed.max()) + Tq - 1
     A.split_reserve(B * Tq, NQ, max_pos + 1, HD)
     # split chunk: a free parameter for tree verify (config 5 names none); with per-sequence chunk cuts 640 keys
-    # measured fastest (256: 166, 384: 149, 512: 147-150, 640: 140, 768: 144, 1024: 154 us per call)
+    # and 1024 measured fastest (256: 174, 384: 158, 512: 147, 640: 136, 768: 143, 1024: 134 us per call)
     chunk = int(os.environ.get("BENCH_TREE_CHUNK", "640"))
     # 0: per-sequence chunks (the library default, batch-invariant), 1: equal runs over the batch
     prev = A.verify_runs(int(os.environ.get("BENCH_VERIFY_RUNS", "0")) if runs is None else runs)
