@@ -134,7 +134,7 @@ __device__ __forceinline__ void lds_wait(T (&r)[N]) {
 // One work item: the rows of tile (or pair) qi from the last of (sequence, KV head) over key split sp. Verify runs call it
 // for the splits [c0, c1) in turn: the first call loads the Q fragments qop, each call but the last requests the first step
 // of the next split before it merges.
-template <int HD, int RB, int RG, int KG_, int NSUB, int KVT, int QT, int OT, bool VER>
+template <int HD, int RB, int RG, int KG_, int NSUB, int KVT, int QT, int OT, bool VER, bool FAR>
 __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh, int qi, int sp, int c0, int c1,
                                              u32x4 (&qop)[RB][HD / 32], unsigned char *smem) {
     using Cf = PrefCfg<HD, RB, RG, KG_, NSUB>;
@@ -197,33 +197,48 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
         if constexpr (XORU) return (ld_voff[0] ^ (unsigned)(vswz(u * RPL) * 8 * sizeof(KE))) + u * RPL * krow_b;
         else return ld_voff[u];
     };
-    // Step k of the walk into stage k % 2. Keys past the last position re-read that position (they are masked), so
-    // every load is in bounds; only a step that crosses the end needs the clamped addresses.
-    // Loads [u0, u1) of the thread's NLD slots (K and V each).
+    // Step k of the walk goes into stage k % 2.
     // 16-bit caches: buffer loads straight into LDS over the byte range the workgroup may read (the ring, or the
     // keys below hi_b), so the rows past the last key of a step read as zeros (they are masked) without clamping.
-    // (Verify runs on a ring may end before it was ever filled: their lanes past the last key are sent out of range.)
-    const uint32_t kv_bytes = p.kv_cap > 0 ? (uint32_t)p.kv_cap * krow_b
-                                           : (uint32_t)(max(hi_b, 1) - 1) * krow_b + (uint32_t)(HD * sizeof(KE));
-    const __amdgpu_buffer_rsrc_t krs = make_rsrc(Kb, kv_bytes), vrs = make_rsrc(Vb, kv_bytes);
+    // (Verify runs on a ring may end before it was ever filled: their range ends at the last key as well.)
+    // fp32 caches: rows past the last key re-read that row, so every load is in bounds.
+    // Byte offsets have 32 bits. FAR: the range is that of one step, at a 64-bit address. Otherwise one range from the start of
+    // the sequence serves every step (host: below 4 GiB): forming it per step cost prompts 1-3% (T = 1024 of 16 q-heads over 8
+    // 26.1 -> 26.9 us), verify runs nothing (16 trees of 8 nodes 129.4 -> 128.1 us).
+    const uint32_t kv_bytes = FAR ? 0u : p.kv_cap > 0 ? (uint32_t)p.kv_cap * krow_b
+                                       : (uint32_t)(max(hi_b, 1) - 1) * krow_b + (uint32_t)(HD * sizeof(KE));
+    const __amdgpu_buffer_rsrc_t krs = make_rsrc(Kb, kv_bytes), vrs = make_rsrc(Vb, kv_bytes);      // !FAR
     int it_cur = 0;                                                     // the step being computed
     // Step k < 0 is a no-op step: every lane is out of range, so its loads write zeros into the stage of the step
     // before (already consumed by every wave) and touch no memory; this keeps the issue points branch-free.
-    // prep(k) forms a step's first byte offset and stages; issue_part(st, u0, u1) issues slots [u0, u1).
-    struct StepLd { unsigned char *kd, *vd; unsigned soff; int s, keys; };
-    auto prep = [&](int k) {
+    // prep(k) forms a step's range, first byte offset and stages; issue_part(st, u0, u1) issues slots [u0, u1) of the thread's
+    // NLD (K and V each).
+    struct StepLd { unsigned char *kd, *vd; const char *k, *v; uint32_t bytes, soff; int s; };
+    auto step_ld = [&](int s, int stage, bool real) {
         StepLd st;
-        const int kst = k < 0 ? it_cur + 1 : k;
-        st.s = s0 + kst;
-        if constexpr (VER) st.keys = p.kv_cap > 0 ? hi_b - st.s * SK : SK;
-        st.kd = smem + (size_t)(kst % 2) * Cf::STAGE;
+        st.s = s;
+        st.kd = smem + (size_t)stage * Cf::STAGE;
         st.vd = st.kd + Cf::HALF;
-        // (the range check covers the vector offset, which holds the step's offset too)
-        st.soff = k < 0 ? kv_bytes : (unsigned)__builtin_amdgcn_readfirstlane((int)((unsigned)key_row(p, st.s * SK) * krow_b));
+        if constexpr (FAR) {
+            const size_t off = (size_t)(unsigned)__builtin_amdgcn_readfirstlane(key_row(p, s * SK)) * krow_b;
+            const int rows = p.kv_cap > 0 && !VER ? SK : min(SK, hi_b - s * SK);
+            st.k = reinterpret_cast<const char *>(Kb) + off;
+            st.v = reinterpret_cast<const char *>(Vb) + off;
+            st.bytes = real && rows > 0 ? (uint32_t)(rows - 1) * krow_b + (uint32_t)(HD * sizeof(KE)) : 0u;
+        } else {
+            // (the range check covers the vector offset, which holds the step's offset too)
+            st.soff = !real ? kv_bytes : (unsigned)__builtin_amdgcn_readfirstlane((int)((unsigned)key_row(p, s * SK) * krow_b));
+        }
         return st;
     };
+    auto prep = [&](int k) {
+        const int kst = k < 0 ? it_cur + 1 : k;
+        return step_ld(s0 + kst, kst % 2, k >= 0);
+    };
     auto issue_part = [&](const StepLd &st, int u0, int u1) {
-        const unsigned row = ld_row + st.soff;
+        unsigned row = ld_row;
+        if constexpr (FAR) asm volatile("" : "+v"(row));                // offsets formed here, not held across the step loop
+        else row += st.soff;
 #pragma unroll
         for (int u = 0; u < NLD; u++) {
             if (u < u0 || u >= u1) continue;
@@ -231,18 +246,21 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
             if (Cf::NLR % Cf::NW != 0 && i >= Cf::NLR) continue;       // wave-uniform: past the tile
             unsigned koff = k_off(u) + row, voff = v_off(u) + row;
             if constexpr (!DMA) {
-                if (st.soff >= kv_bytes) continue;
+                if (FAR ? st.bytes == 0 : st.soff >= kv_bytes) continue;
                 const int S = i * 64 + lane;
                 if (st.s * SK + SK > hi_b) {
                     const unsigned key = (unsigned)(S / SLOTS), lim = (unsigned)(hi_b - 1 - st.s * SK);
                     if (key > lim) { koff -= (key - lim) * krow_b; voff -= (key - lim) * krow_b; }
                 }
-                *reinterpret_cast<u32x4 *>(st.kd + (size_t)S * 16) = load8_op<KVT, F16>(reinterpret_cast<const KE *>(reinterpret_cast<const char *>(Kb) + koff));
-                *reinterpret_cast<u32x4 *>(st.vd + (size_t)S * 16) = load8_op<KVT, F16>(reinterpret_cast<const KE *>(reinterpret_cast<const char *>(Vb) + voff));
+                const char *kp = FAR ? st.k : reinterpret_cast<const char *>(Kb), *vp = FAR ? st.v : reinterpret_cast<const char *>(Vb);
+                *reinterpret_cast<u32x4 *>(st.kd + (size_t)S * 16) = load8_op<KVT, F16>(reinterpret_cast<const KE *>(kp + koff));
+                *reinterpret_cast<u32x4 *>(st.vd + (size_t)S * 16) = load8_op<KVT, F16>(reinterpret_cast<const KE *>(vp + voff));
+            } else if constexpr (FAR) {
+                buffer_load_lds16<VER>(make_rsrc(st.k, st.bytes), st.kd + (size_t)i * 1024, (int)koff);
+                buffer_load_lds16<VER>(make_rsrc(st.v, st.bytes), st.vd + (size_t)i * 1024, (int)voff);
             } else {
-                if (VER && st.keys < SK && (i * 64 + lane) / SLOTS >= st.keys) koff = voff = kv_bytes;
-                buffer_load_lds16<VER>(krs, st.kd + (size_t)i * 1024, (int)koff);
-                buffer_load_lds16<VER>(vrs, st.vd + (size_t)i * 1024, (int)voff);
+                buffer_load_lds16(krs, st.kd + (size_t)i * 1024, (int)koff);
+                buffer_load_lds16(vrs, st.vd + (size_t)i * 1024, (int)voff);
             }
         }
     };
@@ -556,11 +574,7 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
     for (int rb = 0; rb < RB; rb++) l[rb] = sum_over_groups(l[rb]);
     __syncthreads();                                                 // every wave is done with the K/V tiles
     if (VER && sp + 1 < c1) {
-        StepLd nx;
-        nx.s = max(win_lo(pbase + tok0[0], p.window), (sp + 1) * a.kv_split) / SK; nx.kd = smem; nx.vd = smem + Cf::HALF;
-        nx.keys = p.kv_cap > 0 ? hi_b - nx.s * SK : SK;
-        nx.soff = (unsigned)__builtin_amdgcn_readfirstlane((int)((unsigned)key_row(p, nx.s * SK) * krow_b));
-        issue_part(nx, 0, NLD);
+        issue_part(step_ld(max(win_lo(pbase + tok0[0], p.window), (sp + 1) * a.kv_split) / SK, 0, true), 0, NLD);
     }
     if (none) return;
 
@@ -569,14 +583,18 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
     // accumulator in LDS; after one barrier every lane derives M = max m and L = sum l 2^(m - M) (key groups in order) and
     // sums its own blocks over the key groups in order 0..KG-1 (the same order for every row and tiling), each scaled by
     // 2^(m - M) / L (2^(m - M) for a split partial).
+    // Verify runs: the merge's addresses are formed again for every chunk; hoisted out of the chunk loop they were held (spilled,
+    // at HD 128) through the steps (16 sequences x 10 tokens of 16 q-heads over 4 of 128, 256-key chunks: 42.5 -> 41.0 us).
+    int lm = ln, gm = g;
+    if constexpr (VER) asm volatile("" : "+v"(lm), "+v"(gm));
     const int NQ = p.NQ;
-    if (g == 0) {
+    if (gm == 0) {
 #pragma unroll
-        for (int rb = 0; rb < RB; rb++) { stm[wave * RB * 16 + rb * 16 + ln] = m[rb]; stl[wave * RB * 16 + rb * 16 + ln] = l[rb]; }
+        for (int rb = 0; rb < RB; rb++) { stm[wave * RB * 16 + rb * 16 + lm] = m[rb]; stl[wave * RB * 16 + rb * 16 + lm] = l[rb]; }
     }
     float *xb = reinterpret_cast<float *>(xmem);                        // exchange (reuses the tiles)
     auto xslot = [&](int rb, int owner, int sender) {
-        return xb + ((((size_t)(rb * RG + rg) * KG + owner) * (KG - 1) + (sender < owner ? sender : sender - 1)) * 16 + ln) * Cf::XSTR + 4 * g;
+        return xb + ((((size_t)(rb * RG + rg) * KG + owner) * (KG - 1) + (sender < owner ? sender : sender - 1)) * 16 + lm) * Cf::XSTR + 4 * gm;
     };
     // park the blocks of the other owners (constant indices keep acc in registers)
 #pragma unroll
@@ -594,20 +612,20 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
     for (int rb = 0; rb < RB; rb++) {
         float M = kNegInf, mk[KG];
 #pragma unroll
-        for (int k = 0; k < KG; k++) { mk[k] = stm[(rg * KG + k) * RB * 16 + rb * 16 + ln]; M = fmaxf(M, mk[k]); }
+        for (int k = 0; k < KG; k++) { mk[k] = stm[(rg * KG + k) * RB * 16 + rb * 16 + lm]; M = fmaxf(M, mk[k]); }
         float L = 0.f;
 #pragma unroll
         for (int k = 0; k < KG; k++) {
             f[rb][k] = mk[k] == kNegInf ? 0.f : fast_exp2(mk[k] - M);
-            if (mk[k] != kNegInf) L += stl[(rg * KG + k) * RB * 16 + rb * 16 + ln] * f[rb][k];
+            if (mk[k] != kNegInf) L += stl[(rg * KG + k) * RB * 16 + rb * 16 + lm] * f[rb][k];
         }
         if (a.kv_split <= 0) {
             const float inv = L > 0.f ? 1.f / L : 0.f;
 #pragma unroll
             for (int k = 0; k < KG; k++) f[rb][k] *= inv;
         }
-        const int rho = lrow[rb] + ln;
-        if (kg == 0 && g == 0 && rho < hrows) {
+        const int rho = lrow[rb] + lm;
+        if (kg == 0 && gm == 0 && rho < hrows) {
             const int t = tok_of(rho), r = seq * p.T + htok + t, h = kvh * GRP + rho - t * GRP;
             if (a.kv_split > 0) {
                 const size_t pi = ((size_t)r * NQ + h) * a.part.ns_cap + sp;
@@ -619,7 +637,7 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
     }
 #pragma unroll
     for (int rb = 0; rb < RB; rb++) {
-        const int rho = lrow[rb] + ln;
+        const int rho = lrow[rb] + lm;
         if (rho >= hrows) continue;
         const int t = tok_of(rho);
         const size_t ro = (size_t)(seq * p.T + htok + t) * NQ + kvh * GRP + rho - t * GRP;     // output row
@@ -634,7 +652,7 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
                     const f32x4 x = (k == O ? acc[rb][O * DO + j] : *reinterpret_cast<const f32x4 *>(xslot(rb, O, k) + 16 * j)) * f[rb][k];
                     o = k == 0 ? x : o + x;
                 }
-                const int d = 16 * (O * DO + j) + 4 * g;
+                const int d = 16 * (O * DO + j) + 4 * gm;
                 if (a.kv_split > 0) {
                     *reinterpret_cast<f32x4 *>(a.part.acc + (ro * a.part.ns_cap + sp) * HD + d) = o;
                 } else if constexpr (OT == DT_FP32) {
@@ -648,7 +666,7 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
     }
 }
 
-template <int HD, int RB, int RG, int KG_, int NSUB, int WPE, int KVT, int QT, int OT, bool VER>
+template <int HD, int RB, int RG, int KG_, int NSUB, int WPE, int KVT, int QT, int OT, bool VER, bool FAR>
 __global__ void __launch_bounds__(RG * KG_ * 64) __attribute__((amdgpu_waves_per_eu(WPE)))
 prefill_kernel(const PrefArgs a) {
     extern __shared__ __align__(16) unsigned char smem[];
@@ -662,7 +680,7 @@ prefill_kernel(const PrefArgs a) {
         seq = __builtin_amdgcn_readfirstlane(seq); c0 = __builtin_amdgcn_readfirstlane(c0); c1 = __builtin_amdgcn_readfirstlane(c1);
         qi = x / p.NKV; kvh = x - qi * p.NKV;
         u32x4 qop[RB][HD / 32];
-        for (int sp = c0; sp < c1; sp++) prefill_item<HD, RB, RG, KG_, NSUB, KVT, QT, OT, true>(a, seq, kvh, qi, sp, c0, c1, qop, smem);
+        for (int sp = c0; sp < c1; sp++) prefill_item<HD, RB, RG, KG_, NSUB, KVT, QT, OT, true, FAR>(a, seq, kvh, qi, sp, c0, c1, qop, smem);
     } else {
         // XCD-aware work index: dispatch slot b runs on XCD b % 8, and the work items of one KV head (longest first) share
         // an XCD, so that head's K/V stays in one L2. Fewer heads than XCDs: a head's items are dealt in turn to its
@@ -682,7 +700,7 @@ prefill_kernel(const PrefArgs a) {
         seq = p.nseq > 1 ? head / p.NKV : 0; kvh = head - seq * p.NKV;
         qi = a.nsplit > 1 ? item / a.nsplit : item;
         u32x4 qop[RB][HD / 32];
-        prefill_item<HD, RB, RG, KG_, NSUB, KVT, QT, OT, false>(a, seq, kvh, qi, item - qi * a.nsplit, 0, 0, qop, smem);
+        prefill_item<HD, RB, RG, KG_, NSUB, KVT, QT, OT, false, FAR>(a, seq, kvh, qi, item - qi * a.nsplit, 0, 0, qop, smem);
     }
 }
 
@@ -715,12 +733,12 @@ template <int HD, int W>
 using PrefTileCfg = PrefCfg<HD, PrefTile<HD, W>::RB, PrefTile<HD, W>::RG, PrefTile<HD, W>::KG,
                             PrefTile<HD, W>::NSUB>;
 
-template <int HD, int W, int KVT, int QT, int OT, bool VER = false>
+template <int HD, int W, int KVT, int QT, int OT, bool VER = false, bool FAR = VER>
 static hipError_t launch_pref_t(const PrefArgs &a, dim3 grid, hipStream_t st) {
     using T = PrefTile<HD, W>;
     using Cf = PrefTileCfg<HD, W>;
     static bool configured = false;
-    auto kern = prefill_kernel<HD, T::RB, T::RG, T::KG, T::NSUB, T::WPE, KVT, QT, OT, VER>;
+    auto kern = prefill_kernel<HD, T::RB, T::RG, T::KG, T::NSUB, T::WPE, KVT, QT, OT, VER, FAR>;
     if (!configured) {
         hipError_t e = hipFuncSetAttribute(reinterpret_cast<const void *>(kern),
                                            hipFuncAttributeMaxDynamicSharedMemorySize, (int)Cf::lds(VER));
@@ -731,8 +749,19 @@ static hipError_t launch_pref_t(const PrefArgs &a, dim3 grid, hipStream_t st) {
     return hipGetLastError();
 }
 
+// Whether a sequence's K (or V) rows, plus the largest offset inside a step past them, pass 32-bit byte offsets: the narrow
+// tiles have a form that addresses each step in 64 bits.
+static bool pref_far(const Problem &p) {
+    const long long rows = p.kv_cap > 0 ? p.kv_cap : (long long)p.max_pos + 1;
+    return (rows + 128) * p.NKV * p.HD * (p.kv_dtype == DT_FP32 ? 4 : 2) >= 1ll << 32;
+}
+
 template <int KVT, int QT, int OT>
 static hipError_t pref_dispatch_hd(const PrefArgs &a, int wide, dim3 grid, hipStream_t st) {
+    if (pref_far(a.p))
+        return a.p.HD == 128 ? launch_pref_t<128, 0, KVT, QT, OT, false, true>(a, grid, st)
+             : a.p.HD == 256 ? launch_pref_t<256, 0, KVT, QT, OT, false, true>(a, grid, st)
+             : a.p.HD == 512 ? launch_pref_t<512, 0, KVT, QT, OT, false, true>(a, grid, st) : hipErrorInvalidValue;
     switch (a.p.HD) {
     case 128: return launch_pref_t<128, 0, KVT, QT, OT>(a, grid, st);
     case 256:
@@ -861,7 +890,7 @@ static PrefPlan choose_plan(const Problem &p, int kv_split, int nsplit, int ncu)
         if (c < cost) { cost = c; best = pl; }
     };
     if (causal) consider(s0, pref_plan(s0, 0, GRP, p.T, false, false));
-    if (p.HD == 256 && p.kv_dtype != DT_FP32)
+    if (p.HD == 256 && p.kv_dtype != DT_FP32 && !pref_far(p))
         for (int w = 1; w <= 2; w++) {
             const PrefShape sh = pref_shape(256, w);
             consider(sh, pref_plan(sh, w, GRP, p.T, false, false));
