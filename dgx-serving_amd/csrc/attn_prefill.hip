@@ -200,7 +200,8 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
     // Step k of the walk goes into stage k % 2.
     // 16-bit caches: buffer loads straight into LDS over the byte range the workgroup may read (the ring, or the
     // keys below hi_b), so the rows past the last key of a step read as zeros (they are masked) without clamping.
-    // (Verify runs on a ring may end before it was ever filled: their range ends at the last key as well.)
+    // (Verify runs hold to the keys [j_lo, j_hi) of the chunk on both sides: a ring may end before it was ever filled, and a
+    // cache may be filled from the window on only. Rows below the range get offsets below zero, which are out of range too.)
     // fp32 caches: rows past the last key re-read that row, so every load is in bounds.
     // Byte offsets have 32 bits. FAR: the range is that of one step, at a 64-bit address. Otherwise one range from the start of
     // the sequence serves every step (host: below 4 GiB): forming it per step cost prompts 1-3% (T = 1024 of 16 q-heads over 8
@@ -211,20 +212,21 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
     int it_cur = 0;                                                     // the step being computed
     // Step k < 0 is a no-op step: every lane is out of range, so its loads write zeros into the stage of the step
     // before (already consumed by every wave) and touch no memory; this keeps the issue points branch-free.
-    // prep(k) forms a step's range, first byte offset and stages; issue_part(st, u0, u1) issues slots [u0, u1) of the thread's
-    // NLD (K and V each).
+    // step_ld forms a step's range (FAR: rows r0 .. of the step, below key hi), first byte offset and stages; issue_part issues
+    // slots [u0, u1) of the thread's NLD (K and V each).
     struct StepLd { unsigned char *kd, *vd; const char *k, *v; uint32_t bytes, soff; int s; };
-    auto step_ld = [&](int s, int stage, bool real) {
+    auto step_ld = [&](int s, int stage, bool real, int r0, int hi) {
         StepLd st;
         st.s = s;
         st.kd = smem + (size_t)stage * Cf::STAGE;
         st.vd = st.kd + Cf::HALF;
         if constexpr (FAR) {
-            const size_t off = (size_t)(unsigned)__builtin_amdgcn_readfirstlane(key_row(p, s * SK)) * krow_b;
-            const int rows = p.kv_cap > 0 && !VER ? SK : min(SK, hi_b - s * SK);
+            const size_t off = (size_t)(unsigned)__builtin_amdgcn_readfirstlane(key_row(p, s * SK) + r0) * krow_b;
+            const int rows = (p.kv_cap > 0 && !VER ? SK : min(SK, hi - s * SK)) - r0;
             st.k = reinterpret_cast<const char *>(Kb) + off;
             st.v = reinterpret_cast<const char *>(Vb) + off;
             st.bytes = real && rows > 0 ? (uint32_t)(rows - 1) * krow_b + (uint32_t)(HD * sizeof(KE)) : 0u;
+            st.soff = 0u - (uint32_t)r0 * krow_b;
         } else {
             // (the range check covers the vector offset, which holds the step's offset too)
             st.soff = !real ? kv_bytes : (unsigned)__builtin_amdgcn_readfirstlane((int)((unsigned)key_row(p, s * SK) * krow_b));
@@ -233,12 +235,11 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
     };
     auto prep = [&](int k) {
         const int kst = k < 0 ? it_cur + 1 : k;
-        return step_ld(s0 + kst, kst % 2, k >= 0);
+        return step_ld(s0 + kst, kst % 2, k >= 0, 0, VER ? j_hi : hi_b);
     };
     auto issue_part = [&](const StepLd &st, int u0, int u1) {
-        unsigned row = ld_row;
+        unsigned row = ld_row + st.soff;
         if constexpr (FAR) asm volatile("" : "+v"(row));                // offsets formed here, not held across the step loop
-        else row += st.soff;
 #pragma unroll
         for (int u = 0; u < NLD; u++) {
             if (u < u0 || u >= u1) continue;
@@ -274,7 +275,7 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
         if (VER) { if (pt == 0) issue_part(st, 0, NLD); }
         else issue_part(st, pt * PPART, min(NLD, (pt + 1) * PPART));
     };
-    if (nsteps > 0 && fresh) issue(0);
+    if (nsteps > 0 && fresh) issue_part(step_ld(s0, 0, true, VER ? j_lo % SK : 0, VER ? j_hi : hi_b), 0, NLD);
 
     // The Q tile goes through LDS as well (16 bytes per lane of whole rows, where fragment loads straight from memory
     // touch 64 bytes of 16 rows each), in the stage that step 1 will fill, in the K layout: 16-byte column c of tile row R
@@ -574,7 +575,8 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
     for (int rb = 0; rb < RB; rb++) l[rb] = sum_over_groups(l[rb]);
     __syncthreads();                                                 // every wave is done with the K/V tiles
     if (VER && sp + 1 < c1) {
-        issue_part(step_ld(max(win_lo(pbase + tok0[0], p.window), (sp + 1) * a.kv_split) / SK, 0, true), 0, NLD);
+        const int lo = max(win_lo(pbase + tok0[0], p.window), (sp + 1) * a.kv_split), hi = min(hi_b, (sp + 2) * a.kv_split);
+        issue_part(step_ld(lo / SK, 0, true, lo % SK, hi), 0, NLD);
     }
     if (none) return;
 

@@ -84,3 +84,31 @@ def test_ring_that_was_never_filled():
     for b in range(B):
         r = _ref(Q[b], K[b], V[b], int(base[b]), W, None)
         assert (O[b] - r).abs().max().item() <= 2e-3        # as above
+
+
+@pytest.mark.parametrize("runs", [0, 1])
+@pytest.mark.parametrize("T,nq,nkv,hd,chunk,cap", [(8, 24, 4, 256, 640, 0), (8, 24, 4, 256, 96, 0), (12, 16, 4, 128, 128, 512),
+                                                   (30, 16, 8, 256, 256, 512), (1, 24, 4, 256, 256, 0)])
+def test_rows_below_the_window_are_not_read(T, nq, nkv, hd, chunk, cap, runs):
+    """A cache (or ring) filled from the first window on only, to whole 16-key blocks: NaN lies below."""
+    W, base = 300, torch.tensor([1000, 333, 2047, 1024], dtype=torch.int32)
+    B, ML = 4, cap or 2304
+    g = torch.Generator(device="cuda").manual_seed(T + chunk)
+    Q = torch.randn(B, T, nq, hd, device="cuda", generator=g).half()
+    kv = [torch.randn(B, 2304, nkv, hd, device="cuda", generator=g).half() for _ in range(2)]
+    K, V = (torch.full((B, ML, nkv, hd), float("nan"), device="cuda").half() for _ in range(2))
+    for b, n in enumerate(base.tolist()):
+        j = torch.arange((n - W + 1) // 16 * 16, n + T, device="cuda")
+        K[b, j % ML], V[b, j % ML] = kv[0][b, j], kv[1][b, j]
+    max_pos = int(base.max()) + T - 1
+    A.split_reserve(B * T * max(1, -(-A.split_chunk() // chunk)), nq, max_pos + 1, hd)
+    O = torch.empty(B, T, nq, hd, device="cuda")
+    prev = A.verify_runs(runs)
+    try:
+        A.attn_batch_ex(Q, O, B, T, nq, nkv, hd, base.cuda(), max_pos, K=K, V=V, kv_stride=ML * nkv * hd, window=W, chunk=chunk,
+                        kv_cap=cap)
+    finally:
+        A.verify_runs(prev)
+    for b in range(B):
+        r = _ref(Q[b], kv[0][b], kv[1][b], int(base[b]), W, None)
+        assert (O[b] - r).abs().max().item() <= 2e-3, f"sequence {b}"        # as above
