@@ -198,16 +198,16 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
         else return ld_voff[u];
     };
     // Step k of the walk goes into stage k % 2.
-    // 16-bit caches: buffer loads straight into LDS over the byte range the workgroup may read (the ring, or the
-    // keys below hi_b), so the rows past the last key of a step read as zeros (they are masked) without clamping.
+    // 16-bit caches: buffer loads straight into LDS over the byte range the workgroup may read (the keys below
+    // hi_b, or a ring that they fill), so the rows past the last key of a step read as zeros (they are masked) without clamping.
     // (Verify runs hold to the keys [j_lo, j_hi) of the chunk on both sides: a ring may end before it was ever filled, and a
     // cache may be filled from the window on only. Rows below the range get offsets below zero, which are out of range too.)
     // fp32 caches: rows past the last key re-read that row, so every load is in bounds.
     // Byte offsets have 32 bits. FAR: the range is that of one step, at a 64-bit address. Otherwise one range from the start of
     // the sequence serves every step (host: below 4 GiB): forming it per step cost prompts 1-3% (T = 1024 of 16 q-heads over 8
     // 26.1 -> 26.9 us), verify runs nothing (16 trees of 8 nodes 129.4 -> 128.1 us).
-    const uint32_t kv_bytes = FAR ? 0u : p.kv_cap > 0 ? (uint32_t)p.kv_cap * krow_b
-                                       : (uint32_t)(max(hi_b, 1) - 1) * krow_b + (uint32_t)(HD * sizeof(KE));
+    const int kv_rows = max(1, p.kv_cap > 0 ? min(p.kv_cap, hi_b) : hi_b);
+    const uint32_t kv_bytes = FAR ? 0u : (uint32_t)(kv_rows - 1) * krow_b + (uint32_t)(HD * sizeof(KE));
     const __amdgpu_buffer_rsrc_t krs = make_rsrc(Kb, kv_bytes), vrs = make_rsrc(Vb, kv_bytes);      // !FAR
     int it_cur = 0;                                                     // the step being computed
     // Step k < 0 is a no-op step: every lane is out of range, so its loads write zeros into the stage of the step
@@ -222,7 +222,7 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
         st.vd = st.kd + Cf::HALF;
         if constexpr (FAR) {
             const size_t off = (size_t)(unsigned)__builtin_amdgcn_readfirstlane(key_row(p, s * SK) + r0) * krow_b;
-            const int rows = (p.kv_cap > 0 && !VER ? SK : min(SK, hi - s * SK)) - r0;
+            const int rows = min(SK, hi - s * SK) - r0;
             st.k = reinterpret_cast<const char *>(Kb) + off;
             st.v = reinterpret_cast<const char *>(Vb) + off;
             st.bytes = real && rows > 0 ? (uint32_t)(rows - 1) * krow_b + (uint32_t)(HD * sizeof(KE)) : 0u;

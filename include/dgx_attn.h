@@ -193,7 +193,8 @@ hipError_t dgx_attn_batch_noalloc(const void *Q, int q_dtype, const void *Kc, co
  *     LSE combine (the reference's separate launch_gate_sigmoid(attn, gate) after attention).
  *   - kv_cap > 0: the caches are ring buffers of kv_cap rows (a multiple of 64) for a sliding window: key j lives in
  *     row j % kv_cap (the sliding-window ring layout of runtime/decode_state_gemma4.h:9-16, kv_cap). Needs
- *     window > 0 and window + Tq - 1 <= kv_cap, so the keys a launch reads never alias.
+ *     window > 0 and window + Tq - 1 <= kv_cap, so the keys a launch reads never alias. Rows that no key
+ *     has reached yet are not read; once a ring has wrapped, its rows may be read whole, as 64-key steps.
  * Same rows, positions and masks as dgx_attn_batch; a row's result is bit-identical to dgx_attn_batch's when Kp,
  * Vp point at the same caches, gate is null and kv_cap is 0 (or the ring holds the same keys). */
 hipError_t dgx_attn_batch_ex(const void *Q, int q_dtype, const void *Kc, const void *Vc, const void *const *Kp,

@@ -71,3 +71,22 @@ def test_ring_validation():
     for cap, win in [(1000, 512), (1024, 0), (1024, 1025)]:   # not a multiple of 64, no window, window > ring
         with pytest.raises(A.HipError):
             A.attn_batch_ex(Q, O, 1, 1, 16, 8, 128, None, 2000, K=K, V=K, kv_stride=0, window=win, kv_cap=cap, base=2000)
+
+
+@pytest.mark.parametrize("hd,nq,nkv,Sq,base", [(256, 16, 8, 13, 0), (256, 16, 8, 100, 0), (256, 24, 4, 333, 60),
+                                               (128, 16, 4, 100, 0), (512, 16, 1, 100, 5), (256, 16, 8, 500, 7)])
+@pytest.mark.parametrize("kvdt,split", [(0, 0), (1, 0), (1, 64), (2, 0)])
+def test_first_prompt_chunk_into_a_ring(hd, nq, nkv, Sq, base, kvdt, split):
+    """The ring's rows past the last key were never written (NaN): same bits as the linear cache of just the keys."""
+    cap, W = 512 if base + Sq <= 512 else 1024, 400 if base + Sq <= 512 else 512
+    W = min(W, cap - Sq + 1)
+    dt = TORCH_DT[kvdt]
+    g = torch.Generator(device="cuda").manual_seed(Sq + hd)
+    Q = torch.randn(Sq, nq, hd, device="cuda", generator=g).to(torch.float32 if kvdt == 0 else dt)
+    K, V = (torch.randn(base + Sq, nkv, hd, device="cuda", generator=g).to(dt) for _ in range(2))
+    Kr, Vr = (torch.full((cap, nkv, hd), float("nan"), device="cuda").to(dt) for _ in range(2))
+    Kr[:base + Sq], Vr[:base + Sq] = K, V
+    O1, O2 = torch.empty_like(Q), torch.empty_like(Q)
+    A.attn_prefill(Q, K, V, O1, 1, Sq, nq, nkv, hd, base=base, window=W, kv_split=split)
+    A.attn_prefill(Q, Kr, Vr, O2, 1, Sq, nq, nkv, hd, base=base, window=W, kv_cap=cap, kv_split=split)
+    assert torch.isfinite(O2.float()).all() and torch.equal(O1, O2)
