@@ -131,11 +131,11 @@ __device__ __forceinline__ void lds_wait(T (&r)[N]) {
                      "+v"(r[6]), "+v"(r[7]) : [c] "n"(CNT) : "memory");
 }
 
-// One work item: the rows of tile (or pair) qi from the last of (sequence, KV head) over key split sp. Verify runs call it
-// for the splits [c0, c1) in turn: the first call loads the Q fragments qop, each call but the last requests the first step
+// One work item: the rows of tile (or pair) qi from the last of (sequence, KV head) over key split sp. Verify runs (whose
+// sequence is at position p0) call it for the splits [c0, c1) in turn: the first call loads the Q fragments qop, each call but the last requests the first step
 // of the next split before it merges.
 template <int HD, int RB, int RG, int KG_, int NSUB, int KVT, int QT, int OT, bool VER, bool FAR>
-__device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh, int qi, int sp, int c0, int c1,
+__device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int p0, int kvh, int qi, int sp, int c0, int c1,
                                              u32x4 (&qop)[RB][HD / 32], unsigned char *smem) {
     using Cf = PrefCfg<HD, RB, RG, KG_, NSUB>;
     constexpr int KG = Cf::KG, SK = Cf::SK, KS = Cf::KS, DB = Cf::DB, NLD = Cf::NLD, DO = Cf::DO;
@@ -157,10 +157,11 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
     const KE *Kb = kv_base<KE>(p, false, seq) + (size_t)kvh * HD;
     const KE *Vb = kv_base<KE>(p, true, seq) + (size_t)kvh * HD;
     // Prefill tokens are consecutive: token t of this sequence sits at position pbase + t.
-    const int pbase = __builtin_amdgcn_readfirstlane(VER ? tok_pos(p, seq, 0) : p.pos_arr ? p.pos_arr[seq] : p.base);
+    const int pbase = VER ? p0 : __builtin_amdgcn_readfirstlane(p.pos_arr ? p.pos_arr[seq] : p.base);
 
     // The work item's tokens: one tile, or two half tiles (longest first; an empty half has tok1 == tok0).
-    const int ht0 = a.nht - 1 - qi, ht1 = a.pair && qi < ht0 ? qi : -1;
+    const bool pair = !VER && a.pair, split = VER || a.kv_split > 0;    // (verify items are single tiles over one chunk)
+    const int ht0 = a.nht - 1 - qi, ht1 = pair && qi < ht0 ? qi : -1;
     int tok0[2], tok1[2];
     tok0[0] = ht0 * a.tqh; tok1[0] = min(p.T, tok0[0] + a.tqh);
     tok0[1] = ht1 < 0 ? 0 : ht1 * a.tqh; tok1[1] = ht1 < 0 ? 0 : min(p.T, tok0[1] + a.tqh);
@@ -169,7 +170,7 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
     if (tok1[1] > tok0[1]) j_lo = min(j_lo, win_lo(pbase + tok0[1], p.window));
     const int hi_b = pbase + tok1[0];                                   // one past the last key (clamp bound)
     int j_hi = hi_b;
-    if (a.kv_split > 0) { j_lo = max(j_lo, sp * a.kv_split); j_hi = min(j_hi, (sp + 1) * a.kv_split); }
+    if (split) { j_lo = max(j_lo, sp * a.kv_split); j_hi = min(j_hi, (sp + 1) * a.kv_split); }
     const bool fresh = !VER || sp == c0;
     const bool none = VER && j_lo >= j_hi;                              // no row of the tile has keys in this chunk
     const int s0 = j_lo / SK, nsteps = j_lo < j_hi ? (j_hi - 1) / SK - s0 + 1 : 0;
@@ -287,7 +288,7 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
         f32x4 raw[QDMA ? 1 : Cf::NQL][2];
 #pragma unroll
         for (int u = 0; u < Cf::NQL; u++) {
-            const int i = wave * Cf::NQL + u, hb = a.pair && i * RPL >= HR ? 1 : 0;
+            const int i = wave * Cf::NQL + u, hb = pair && i * RPL >= HR ? 1 : 0;
             const int R = i * RPL + lane / SLOTS, rho = R - hb * HR, nr = (tok1[hb] - tok0[hb]) * GRP;
             const int off = (rho + tok_of(rho) * (p.NQ - GRP)) * HD + ((lane % SLOTS) ^ kswz(R)) * 8;
             const QE *qb = reinterpret_cast<const QE *>(p.Q) + ((size_t)(seq * p.T + tok0[hb]) * p.NQ + kvh * GRP) * HD;
@@ -317,7 +318,7 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
     // This wave's row blocks: block rb covers rows [lrow[rb], lrow[rb] + 16) of half tile hb. Positions per row (an invalid
     // row has pos = -1 and attends nothing), and the wave-uniform key span of each block (positions grow with the row's
     // token).
-    const int hb = a.pair ? rg * RB * 16 / HR : 0;
+    const int hb = pair ? rg * RB * 16 / HR : 0;
     const int htok = tok0[hb], hrows = (tok1[hb] - tok0[hb]) * GRP;
     int lrow[RB], rpos[RB];
     uint32_t anc[RB];                                                   // verify: tree masks of the rows (relative to pbase)
@@ -621,7 +622,7 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
             f[rb][k] = mk[k] == kNegInf ? 0.f : fast_exp2(mk[k] - M);
             if (mk[k] != kNegInf) L += stl[(rg * KG + k) * RB * 16 + rb * 16 + lm] * f[rb][k];
         }
-        if (a.kv_split <= 0) {
+        if (!split) {
             const float inv = L > 0.f ? 1.f / L : 0.f;
 #pragma unroll
             for (int k = 0; k < KG; k++) f[rb][k] *= inv;
@@ -629,7 +630,7 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
         const int rho = lrow[rb] + lm;
         if (kg == 0 && gm == 0 && rho < hrows) {
             const int t = tok_of(rho), r = seq * p.T + htok + t, h = kvh * GRP + rho - t * GRP;
-            if (a.kv_split > 0) {
+            if (split) {
                 const size_t pi = ((size_t)r * NQ + h) * a.part.ns_cap + sp;
                 a.part.m[pi] = M; a.part.l[pi] = L;
             } else if (p.lse) {
@@ -655,7 +656,7 @@ __device__ __forceinline__ void prefill_item(const PrefArgs &a, int seq, int kvh
                     o = k == 0 ? x : o + x;
                 }
                 const int d = 16 * (O * DO + j) + 4 * gm;
-                if (a.kv_split > 0) {
+                if (split) {
                     *reinterpret_cast<f32x4 *>(a.part.acc + (ro * a.part.ns_cap + sp) * HD + d) = o;
                 } else if constexpr (OT == DT_FP32) {
                     *reinterpret_cast<f32x4 *>(reinterpret_cast<float *>(p.O) + ro * HD + d) = o;
@@ -675,14 +676,27 @@ prefill_kernel(const PrefArgs a) {
     const Problem &p = a.p;
     int seq, kvh, qi;                                                   // sequence, KV head, tile from the last
     if constexpr (VER) {
-        // Verify: runs of a sequence's key chunks, KV heads and tiles of one run side by side.
+        // Verify: runs of key chunks, KV heads and tiles of one run side by side.
         const int per = p.NKV * a.nht, it = (int)blockIdx.x / per, x = (int)blockIdx.x - it * per;
-        int c0, c1;
-        if (!find_run(p, a.kv_split, a.split_m, it, a.slots, seq, c0, c1)) return;
-        seq = __builtin_amdgcn_readfirstlane(seq); c0 = __builtin_amdgcn_readfirstlane(c0); c1 = __builtin_amdgcn_readfirstlane(c1);
+        int p0, c0, c_end, left;
+        if (!find_run(p, a.kv_split, a.split_m, it, a.slots, seq, p0, c0, c_end, left)) return;
         qi = x / p.NKV; kvh = x - qi * p.NKV;
-        u32x4 qop[RB][HD / 32];
-        for (int sp = c0; sp < c1; sp++) prefill_item<HD, RB, RG, KG_, NSUB, KVT, QT, OT, true, FAR>(a, seq, kvh, qi, sp, c0, c1, qop, smem);
+        for (;;) {
+            seq = __builtin_amdgcn_readfirstlane(seq); c0 = __builtin_amdgcn_readfirstlane(c0);
+            p0 = __builtin_amdgcn_readfirstlane(p0);
+            const int c1 = __builtin_amdgcn_readfirstlane(min(c_end, c0 + left));
+            u32x4 qop[RB][HD / 32];
+            for (int sp = c0; sp < c1; sp++) prefill_item<HD, RB, RG, KG_, NSUB, KVT, QT, OT, true, FAR>(a, seq, p0, kvh, qi, sp, c0, c1, qop, smem);
+            left -= c1 - c0;
+            if (left <= 0) return;
+            int n;
+            do {                                                        // the next sequence with keys
+                if (++seq >= p.nseq) return;                            // (unreachable while the counts agree)
+                seq_chunks(p, a.kv_split, a.split_m, seq, p0, c0, n);
+            } while (n <= 0);
+            c_end = c0 + n;
+            __syncthreads();                                            // every wave is done with the merge's LDS
+        }
     } else {
         // XCD-aware work index: dispatch slot b runs on XCD b % 8, and the work items of one KV head (longest first) share
         // an XCD, so that head's K/V stays in one L2. Fewer heads than XCDs: a head's items are dealt in turn to its
@@ -702,7 +716,7 @@ prefill_kernel(const PrefArgs a) {
         seq = p.nseq > 1 ? head / p.NKV : 0; kvh = head - seq * p.NKV;
         qi = a.nsplit > 1 ? item / a.nsplit : item;
         u32x4 qop[RB][HD / 32];
-        prefill_item<HD, RB, RG, KG_, NSUB, KVT, QT, OT, false, FAR>(a, seq, kvh, qi, item - qi * a.nsplit, 0, 0, qop, smem);
+        prefill_item<HD, RB, RG, KG_, NSUB, KVT, QT, OT, false, FAR>(a, seq, 0, kvh, qi, item - qi * a.nsplit, 0, 0, qop, smem);
     }
 }
 
@@ -954,11 +968,23 @@ hipError_t launch_verify_tile(const Problem &p, int chunk, const Partials &part,
     if (p.max_pos / chunk + 1 > part.ns_cap) return hipErrorInvalidValue;
     const int GRP = p.NQ / p.NKV;
     const int tq = 64 / GRP, nt = (p.T + tq - 1) / tq;
-    const long long wgs = chunk_items_bound(p, chunk) * p.NKV * nt;
+    // Runs per (KV head, tile): as many as are resident at once, or of two to four rounds, where one leaves the device less
+    // full. Their number bounds the grid: a workgroup without work still takes its LDS and reads the positions (about 1 us).
+    const long long per = (long long)p.NKV * nt, res = std::max(1, device_cus()) * (p.HD == 128 ? 2 : 1);
+    long long runs = 1;
+    double use = 0.;
+    for (int m = 1; m <= 4 && use < 0.9; m++) {
+        const long long r = std::max(1ll, m * res / per), rounds = (r * per + res - 1) / res;
+        const double u = (double)(r * per) / (double)(rounds * res);
+        if (u > use) { use = u; runs = r; }
+    }
+    const long long wgs = std::min(chunk_items_bound(p, chunk), runs) * per;
     if (wgs > INT_MAX) return hipErrorInvalidConfiguration;
-    PrefArgs a{p, part, chunk, div_magic(chunk), nt, 1, tq, 0, 0, p.nseq * p.NKV, GRP, p.scale * kLog2e, 0,
+    Problem pr = p;
+    if (p.pos_mode == 1) pr.pos_step = 0;                              // see seq_chunks
+    PrefArgs a{pr, part, chunk, div_magic(chunk), nt, 1, tq, 0, 0, p.nseq * p.NKV, GRP, p.scale * kLog2e, 0,
                (reinterpret_cast<uintptr_t>(p.Q) & 15) == 0 ? 1 : 0, 65535 / GRP + 1,
-               std::max(1, device_cus() * (p.HD == 128 ? 2 : 1) / (p.NKV * nt)), 0};
+               (int)runs, 0};
     const dim3 grid((unsigned)wgs);
     const bool q32 = p.q_dtype == DT_FP32;
     if (p.kv_dtype == DT_F16)

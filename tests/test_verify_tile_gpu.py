@@ -1,6 +1,6 @@
 """Verify and tree runs on the tile kernel: edges of the tiles (16-row blocks, 32 and 64 rows, several token tiles), of the
-64-key steps and of the chunks, one to many sequences, against fp32 attention; and the device's enumeration of the chunk
-items against a count on the host."""
+64-key steps and of the chunks, one to many sequences, against fp32 attention; runs over several chunks and sequences against
+each sequence alone."""
 import numpy as np
 import pytest
 import torch
@@ -31,7 +31,7 @@ def _ref(Q, K, V, base, window, anc):
     return out
 
 
-# T x GRP rows: 17 (one past a block), 32, 33 (past the narrow tile), 48, 64, 65 and 96 (two token tiles), 200, 36 (GRP 36)
+# T x GRP rows: 17 (one past a block), 32, 33, 48, 64, 65 and 96 (two token tiles), 200, 36 (GRP 36)
 SHAPES = [(17, 1, 1, 256), (16, 2, 1, 128), (11, 6, 2, 256), (8, 24, 4, 256), (16, 16, 4, 128), (13, 10, 2, 256),
           (16, 24, 4, 256), (25, 16, 2, 128), (1, 36, 1, 256)]
 # 24 sequences of 64-key chunks are more items than run at once: a workgroup takes several chunks in turn; 70 sequences
@@ -112,3 +112,32 @@ def test_rows_below_the_window_are_not_read(T, nq, nkv, hd, chunk, cap, runs):
     for b in range(B):
         r = _ref(Q[b], kv[0][b], kv[1][b], int(base[b]), W, None)
         assert (O[b] - r).abs().max().item() <= 2e-3, f"sequence {b}"        # as above
+
+
+# Workgroups at once: 256 (HD 256) or 512 (HD 128) over KV heads x tiles. Chunks that outnumber them, with more or fewer
+# sequences than runs, and a count of KV heads x tiles that does not divide the device.
+@pytest.mark.parametrize("B,T,nq,nkv,hd,chunk,hi,window", [
+    (40, 8, 24, 4, 256, 64, 900, 0), (64, 8, 24, 4, 256, 64, 600, 0), (65, 8, 24, 4, 256, 64, 600, 0),
+    (130, 9, 16, 4, 128, 64, 700, 0), (9, 30, 24, 3, 256, 96, 2000, 0), (33, 20, 16, 8, 256, 64, 900, 300),
+    (3, 32, 48, 24, 256, 64, 500, 0), (2, 8, 24, 4, 256, 64, 9000, 0), (5, 1, 40, 1, 256, 32, 9000, 0)])
+def test_runs_do_not_show_in_the_bits(B, T, nq, nkv, hd, chunk, hi, window):
+    rng = np.random.default_rng(B)
+    base = rng.integers(0, hi, B).astype(np.int32)
+    base[rng.integers(0, B, B // 3)] = 0                    # several one-chunk sequences
+    base[B // 2] = hi
+    ML, max_pos = hi + T, hi + T - 1
+    g = torch.Generator(device="cuda").manual_seed(B + T)
+    Q = torch.randn(B, T, nq, hd, device="cuda", generator=g).half()
+    K, V = (torch.randn(B, ML, nkv, hd, device="cuda", generator=g).half() for _ in range(2))
+    A.split_reserve(B * T * -(-A.split_chunk() // chunk), nq, max_pos + 1, hd)
+    O, lse = torch.full((B, T, nq, hd), float("nan"), device="cuda"), torch.full((B, T, nq), float("nan"), device="cuda")
+    A.attn_batch(Q, K, V, O, B, T, nq, nkv, hd, torch.from_numpy(base).cuda(), ML * nkv * hd, max_pos, chunk=chunk, window=window,
+                 lse=lse)
+    assert torch.isfinite(O).all() and torch.isfinite(lse).all(), "a row was not written"
+    for b in range(B):
+        Ob, lb = torch.empty_like(O[b]), torch.empty_like(lse[b])
+        A.attn_batch(Q[b], K[b], V[b], Ob, 1, T, nq, nkv, hd, torch.from_numpy(base[b:b + 1]).cuda(), 0, int(base[b]) + T - 1,
+                     chunk=chunk, window=window, lse=lb)
+        assert torch.equal(O[b], Ob) and torch.equal(lse[b], lb), f"sequence {b} at {base[b]}"
+    r = _ref(Q[B // 2], K[B // 2], V[B // 2], hi, window, None)
+    assert (O[B // 2] - r).abs().max().item() <= 2e-3       # as above
