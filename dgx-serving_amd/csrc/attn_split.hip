@@ -276,10 +276,13 @@ struct SplitCfg {
 };
 
 
-// NT: non-temporal K/V loads, for caches that one workgroup reads once (one token tile, no cache shared by the rows) and
-// that may exceed the 256 MB last-level cache. The 8-sequence HD 512 decode (up to 32K keys, 376 MB) takes 81.4 us with them
-// against 89.0 with plain loads; 6 sequences of up to 4.3K keys, whose caches stay in the last level, 44.2 against 40.5.
-// Rows that share a cache (kv_stride 0) keep the plain loads as well: the L2 serves their repeats.
+// NT: non-temporal K/V loads, for 16-bit HD 512 caches that one workgroup reads once (one token tile, no cache shared by the
+// rows) and that may exceed the 256 MB last-level cache. The 8-sequence HD 512 decode (up to 32K keys, 376 MB) takes 82.2 us
+// with them against 89.9 with plain loads. max_pos bounds the caches, so a server that passes its capacity gets these loads for
+// short contexts too: where other data pass through between two calls they cost nothing there (6 sequences of up to 4.3K keys
+// under a capacity of 128K: 58.1 against 58.9 us, 8 of up to 16K: 62.7 against 64.3); a 29 MB cache that nothing displaced
+// reads 43.9 against 40.5. Choosing on the device from the positions kept two load forms in one kernel, more than 256 VGPRs and
+// so one wave per SIMD: 105-110 us. Rows that share a cache (kv_stride 0) keep the plain loads: the L2 serves their repeats.
 template <int HD, int RB, int KVT, int QT, bool NT>
 __global__ void __launch_bounds__(256) split_kernel(const SplitArgs a) {
     using Cf = SplitCfg<HD, RB>;
@@ -878,7 +881,7 @@ static hipError_t launch_split_t(SplitArgs &a, dim3 grid, bool equal_runs, hipSt
             return hipGetLastError();
         }
     }
-    if constexpr (RB == 1) {
+    if constexpr (RB == 1 && HD == 512 && KVT != DT_FP32) {
         // (bound of the keys read: every position up to max_pos, or the window)
         const double keys = a.p.window > 0 ? std::min((double)a.p.max_pos + 1, (double)a.p.window + a.p.T) : (double)a.p.max_pos + 1;
         const double bytes = keys * a.p.nseq * a.p.NKV * HD * 2 * sizeof(typename Elem<KVT>::T);
@@ -891,7 +894,9 @@ static hipError_t launch_split_t(SplitArgs &a, dim3 grid, bool equal_runs, hipSt
 template <int HD, int KVT, int QT>
 static hipError_t dispatch_rb(SplitArgs &a, int RB, dim3 grid, bool eq, hipStream_t st) {
     switch (RB) {
-    case 1: return launch_split_t<HD, 1, KVT, QT>(a, grid, eq, st);
+    case 1:                                            // (16-bit caches at HD 128 and 256: the streaming decode kernel)
+        if constexpr (HD == 512 || KVT == DT_FP32) return launch_split_t<HD, 1, KVT, QT>(a, grid, eq, st);
+        else return hipErrorInvalidValue;
     case 2: return launch_split_t<HD, 2, KVT, QT>(a, grid, eq, st);
     case 3: return launch_split_t<HD, 3, KVT, QT>(a, grid, eq, st);
     case 4: return launch_split_t<HD, 4, KVT, QT>(a, grid, eq, st);
