@@ -280,11 +280,11 @@ static hipError_t launch_dec_e(const DecodeArgs &a, dim3 grid, hipStream_t st) {
 template <int HD, int RW, int KVT, int QT>
 static hipError_t launch_dec_rw(const DecodeArgs &a, dim3 grid, hipStream_t st) {
     // Early refill (the same float operations in the same order) for sliding windows, and at HD 256 for launches of at most
-    // two workgroups per CU of a 256-CU device: there no other wave covers a tile's load. A one-token step of 3 sequences
+    // two workgroups per CU: there no other wave covers a tile's load. A one-token step of 3 sequences
     // over up to 2.9K keys takes 20.8 instead of 23.8 us, 6 over up to 538 29.9 instead of 32.5; the 564-workgroup batch
     // of 16 stays at 57.8 either way, and at HD 128 it gains nothing (13.8 against 13.5 us for one sequence of 512 keys).
     // Two tiles ahead (254 VGPRs, one wave per SIMD) took 22.5 and 31.1 us.
-    if (a.p.window > 0 || (HD == 256 && grid.x <= 512u)) return launch_dec_e<HD, RW, KVT, QT, true>(a, grid, st);
+    if (a.p.window > 0 || (HD == 256 && (int)grid.x <= 2 * device_cus())) return launch_dec_e<HD, RW, KVT, QT, true>(a, grid, st);
     return launch_dec_e<HD, RW, KVT, QT, false>(a, grid, st);
 }
 
@@ -308,7 +308,7 @@ static hipError_t dec_dispatch_hd(const DecodeArgs &a, dim3 grid, int rw, hipStr
 bool decode_stream_supported(const Problem &p) {
     // One 16-row block (RW = 1). The kernel also runs RW = 2..4 row blocks, one wave each per key lane, but then
     // the row waves re-read every tile, which measured slower than the cooperative split kernel on the B=16 x
-    // 8-token tree workload (205 vs 193 us), so those shapes go to the split kernel.
+    // 8-token tree workload (205 vs 193 us), so those shapes go to the verify form of the prefill tile.
     return p.T >= 1 && (p.HD == 128 || p.HD == 256) && p.NQ % p.NKV == 0 && p.T * (p.NQ / p.NKV) <= 16 &&
            p.kv_dtype != DT_FP32;
 }
@@ -557,7 +557,7 @@ hipError_t launch_decode_f32(const Problem &p, int chunk, const Partials &part, 
     // Early refill of a tile's registers for small launches, as in the 16-bit kernel: 1 sequence of 2.9K keys at HD 256 61.5
     // instead of 68.4 us, 4 of up to 1K 61.5 instead of 70.3, 3 of up to 4K at HD 128 37.2 instead of 45.3; the
     // 564-workgroup batch of 16 takes 119 us without it.
-    if (grid.x <= 512u)
+    if ((int)grid.x <= 2 * device_cus())
         return p.HD == 128 ? launch_f32_t<128, true>(a, grid, st) : launch_f32_t<256, true>(a, grid, st);
     return p.HD == 128 ? launch_f32_t<128, false>(a, grid, st) : launch_f32_t<256, false>(a, grid, st);
 }

@@ -203,6 +203,9 @@ __device__ __forceinline__ bool find_run(const Problem &p, int C, uint32_t M, in
     return false;
 }
 
+// CUs of the current device (0: unknown).
+int device_cus();
+
 // Upper bound of the (sequence, chunk) items of a launch: every chunk up to max_pos, or, under a sliding
 // window with consecutive token positions, the at most (window + T - 2) / chunk + 2 chunks a window of window + T - 1
 // keys meets (a 32K-key cache with a 1K window then launches 6 items per sequence and head, not 128).
@@ -229,7 +232,7 @@ hipError_t launch_decode_f32(const Problem &p, int chunk, const Partials &part, 
 // tile writing O directly; kv_split > 0: keys cut at absolute multiples of kv_split, partials + combine.
 hipError_t launch_prefill(const Problem &p, int kv_split, const Partials &part, hipStream_t st);
 // Verify and tree runs on the prefill tile: up to `chunk` keys per work item, partials for launch_combine (16-bit caches,
-// HD 128 / 256, chunk a multiple of 64, consecutive tokens).
+// HD 128 / 256, chunk a multiple of 32, consecutive tokens).
 bool verify_tile_supported(const Problem &p, int chunk);
 hipError_t launch_verify_tile(const Problem &p, int chunk, const Partials &part, hipStream_t st);
 // The key split chosen for kv_split = -1 (0: none).

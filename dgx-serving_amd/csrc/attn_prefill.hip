@@ -821,8 +821,7 @@ size_t prefill_lds_bytes(int HD) {
     }
 }
 
-// CUs of the current device (0: unknown).
-static int device_cus() {
+int device_cus() {
     static std::atomic<int> cus[64];
     int dev = 0;
     if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= 64) return 0;
