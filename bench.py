@@ -1,10 +1,10 @@
-"""Benchmark of the MI355X attention hot path (BASELINE.json metric).
+"""Benchmark of the MI355X attention hot path.
 
-Headline (`value`): batched split-KV decode at BASELINE.json config 2 - B=16, Hq=24, Hkv=4, hd=256, f16 KV cache
+Headline (`value`): batched split-KV decode - B=16, Hq=24, Hkv=4, hd=256, f16 KV cache
 [16, 8192, 4, 256], ragged context lengths L_b ~ U[256, 8192] (seeded), split 512 + LSE combine, one query token
 per sequence - as algorithmic HBM GB/s: bytes = sum_b L_b * Hkv * hd * 2 (K and V) * 2 B + |Q| + |O|.
 Alongside: causal flash prefill at config 3 (T=1024, Hq=16, Hkv=8, hd=256, bf16) as TFLOP/s with
-flops = 4 * hd * Hq * sum of attended keys, and the other BASELINE.json configs in µs per layer call.
+flops = 4 * hd * Hq * sum of attended keys, and the other workloads in µs per layer call.
 A step is one layer call (the split kernel plus the LSE combine kernel for decode).
 
 Timing: W untimed warm-up steps, then exactly K steps between torch.cuda.synchronize() calls, measured with
@@ -129,8 +129,8 @@ def run_tree(steps, warmup, seed=5, runs=None):
     ancd = torch.from_numpy(anc.reshape(-1).view(np.int32)).cuda()
     max_pos = int(committed.max()) + Tq - 1
     A.split_reserve(B * Tq, NQ, max_pos + 1, HD)
-    # split chunk: a free parameter for tree verify (config 5 names none); with per-sequence chunk cuts 640 keys
-    # and 1024 measured fastest (256: 174, 384: 158, 512: 147, 640: 136, 768: 143, 1024: 134 us per call)
+    # split chunk: a free parameter of tree verify; 640 keys is kept so that runs stay comparable, 768 measured fastest
+    # (256: 160, 384: 146, 512: 145, 640: 134, 768: 128, 1024: 132 us per call)
     chunk = int(os.environ.get("BENCH_TREE_CHUNK", "640"))
     # 0: per-sequence chunks (the library default, batch-invariant), 1: equal runs over the batch
     prev = A.verify_runs(int(os.environ.get("BENCH_VERIFY_RUNS", "0")) if runs is None else runs)

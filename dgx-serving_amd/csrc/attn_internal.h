@@ -96,8 +96,8 @@ __device__ __forceinline__ int wave_scan64(int v) {
 // items go last, where they land on the CUs that get a third workgroup (measured: a CU with three full items runs
 // 20% longer than one with two).
 // The divisions by C are multiplications and the scans run on the VALU (2.2 -> about 1 us before a workgroup's first load).
-// A form without the second pass over the positions starts the short items of phase 1 as early as the others, and the
-// 564-workgroup decode batch is then slower (57.9 against 57.5 us).
+// A form without the second pass over the positions took 57.9 against 57.5 us on the 564-workgroup decode batch, which is no
+// more than runs of one build differ by; the two passes are the form that starts the short items no earlier than the others.
 __device__ __forceinline__ bool find_item(const Problem &p, int C, uint32_t M, int rest, int &seq, int &c, int &lo, int &hi) {
     const int lane_ = threadIdx.x & 63, cmax = div_by(p.max_pos, C, M);
     seq = -1; c = 0;

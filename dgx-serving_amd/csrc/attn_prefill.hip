@@ -946,8 +946,8 @@ hipError_t launch_prefill(const Problem &p, int kv_split, const Partials &part, 
 
 // Verify and tree runs (more than 16 rows per KV head): the keys in absolute chunks, found on the device from the positions
 // (find_run), one partial per (row, chunk). Against a tile of four waves that each walk all 16-key tiles of the chunk, two
-// key groups and 64-key steps halve the chain of a chunk: a 7-token draft over 3001 keys (24 workgroups) takes 23.9 instead
-// of 47.1 us. 16 trees of 8 nodes over up to 16K keys (876 chunks, bound by HBM: 26 GB/s per CU inside the loop) take 131
+// key groups and 64-key steps halve the chain of a chunk: a 7-token draft over 3001 keys (24 workgroups) takes 24.3 instead
+// of 47.0 us. 16 trees of 8 nodes over up to 16K keys (876 chunks, bound by HBM: 26 GB/s per CU inside the loop) take 128
 // against 133 us; one chunk per workgroup there 134. 32-key steps took 158 us with two stages (a step then is one HBM
 // latency) and 153 with four.
 bool verify_tile_supported(const Problem &p, int chunk) {

@@ -76,9 +76,9 @@ def _ck(code, what):
         raise HipError(f"{what} failed: hipError {code}")
 
 
-# Every call passes through the two functions below several times, and a decode step makes one call per layer and more: a
-# call that takes 5 us on the host (2.7 of them in torch.cuda.current_stream(), 1.5 in ctypes.c_void_p objects) bounds the
-# short ones. Plain integers and the raw stream handle bring it to 1.6 us.
+# Every call passes through the two functions below several times, and a decode step makes one call per layer and more, so
+# the host's time bounds the short ones. torch.cuda.current_stream() takes 2.9 us, the raw handle 0.3; with it and with plain
+# integers instead of ctypes.c_void_p objects a call of one launch takes 5.8 us on the host instead of 8.4.
 def _ptr(t):
     return None if t is None else t.data_ptr()
 

@@ -179,7 +179,7 @@ hipError_t dgx_attn_batch(const void *Q, int q_dtype, const void *Kc, const void
  * and results as dgx_attn_batch (bit-identical: the same kernels), but the split partials live in a fixed 64 MiB
  * device array inside the library (one per GPU, held until the process ends) instead of the reserved pool, so no
  * dgx_attn_split_reserve is needed. Limit: B * Tq * NQ * (max_pos / chunk + 1) partials of (HD + 2) floats must
- * fit in 64 MiB (e.g. BASELINE config 2 at chunk 512 needs 6.3 MB); larger calls return hipErrorInvalidValue.
+ * fit in 64 MiB (e.g. 16 rows of 24 q-heads of 256 over 8K keys at chunk 512 need 6.3 MB); larger calls return hipErrorInvalidValue.
  * Calls that overlap on one GPU (different streams or host threads) share the array and race; serialize them. */
 hipError_t dgx_attn_batch_noalloc(const void *Q, int q_dtype, const void *Kc, const void *Vc, int kv_dtype, void *O,
                                   int o_dtype, float *lse, int B, int Tq, int NQ, int NKV, int HD, const int *base_b,

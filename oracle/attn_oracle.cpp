@@ -117,7 +117,7 @@ void oracle_gen_xorshift(uint64_t *state, float *out, size_t n) {
     *state = s;
 }
 // Seeded N(mean, sd^2) by Box-Muller over a splitmix64 counter stream (element i depends only on seed and i,
-// so any slice can be regenerated independently). Used for the BASELINE.json configs (Q~N(0,1), K,V~N(0,0.5^2)).
+// so any slice can be regenerated independently). Used for the measured workloads (Q~N(0,1), K,V~N(0,0.5^2)).
 static inline uint64_t splitmix64(uint64_t z) {
     z += 0x9e3779b97f4a7c15ull; z = (z ^ (z >> 30)) * 0xbf58476d1ce4e5b9ull;
     z = (z ^ (z >> 27)) * 0x94d049bb133111ebull; return z ^ (z >> 31);

@@ -1,6 +1,6 @@
 """Shared helpers of the parity tests: seeded inputs, device upload, the CPU oracle call and error metrics.
 
-Tolerances (BASELINE.json north_star): max-abs <= 1e-2 and mean-abs <= 1e-3 on outputs against the fp64 /
+Tolerances: max-abs <= 1e-2 and mean-abs <= 1e-3 on outputs against the fp64 /
 fp32-accumulate reference, LSE within 1e-4 relative.
 """
 import numpy as np

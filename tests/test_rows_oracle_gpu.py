@@ -1,5 +1,4 @@
-"""Oracle parity of the paths whose other tests compare the library with itself, plus BASELINE config 4b at its
-full workload.
+"""Oracle parity of the paths whose other tests compare the library with itself, plus sliding-window decode at full size.
 
 - Config 4b (sliding-window batched decode, the Gemma local layer as models/gemma4_batch.cu:173-174 calls it):
   B=8, context lengths U[1024, 32768] seeded, window 1024, Hq=16 Hkv=8 hd=256, bf16 KV and bf16 Q/O, through

@@ -40,7 +40,7 @@ def _compare(seed, B, Tq, NQ, NKV, HD, ML, lo, chunk, tree):
 
 
 def test_noalloc_decode_two_calls():
-    _compare(1, 16, 1, 24, 4, 256, 8192, 256, 512, False)     # BASELINE config 2 shape
+    _compare(1, 16, 1, 24, 4, 256, 8192, 256, 512, False)     # the batched decode workload
     _compare(2, 3, 1, 24, 4, 256, 2048, 1, 256, False)        # smaller second call
 
 
